@@ -71,6 +71,9 @@ __device__ __forceinline__ constexpr double Mi(int k, int v) {
 // icsr table (utils.hpp:749-767), 0-based; row MTS_NTYPES is the typeless
 // wall link of a buffer cell (full bounce-back: target = opposite).
 __constant__ signed char c_icsr[MTS_NTYPES + 1][9];
+// the same for ic = 1..8 in bits 4(ic-1)..4ic-1 of one word per type
+// (TYPE_NONE takes the typeless row; its sites have no wall link)
+__constant__ uint32_t c_icsr4[64];
 
 // Site helpers ---------------------------------------------------------------
 struct Lat {
@@ -95,20 +98,10 @@ struct Lat {
     }
 };
 
-template <class S>
-struct Store;
-template <>
-struct Store<double> {
-    static constexpr bool dev = false;
-    __device__ __forceinline__ static double ld(const double* a, int64_t i) { return __builtin_nontemporal_load(a + i); }
-    __device__ __forceinline__ static void st(double* a, int64_t i, double v) { __builtin_nontemporal_store(v, a + i); }
-};
-template <>
-struct Store<float> {
-    static constexpr bool dev = true;
-    __device__ __forceinline__ static float ld(const float* a, int64_t i) { return __builtin_nontemporal_load(a + i); }
-    __device__ __forceinline__ static void st(float* a, int64_t i, float v) { __builtin_nontemporal_store(v, a + i); }
-};
+// Populations are read by the neighbours' threads too: loads are cached, stores
+// stream past the caches (the next read is a full step later).
+__device__ __forceinline__ double ld64(const double* __restrict__ a, int64_t i) { return a[i]; }
+__device__ __forceinline__ void st64(double* __restrict__ a, int64_t i, double v) { __builtin_nontemporal_store(v, a + i); }
 
 // ============================================================================
 // FP64 reference-order arithmetic.  The reference evaluates dense 9x9
@@ -245,63 +238,64 @@ __device__ __forceinline__ void source64(double* f, double ux, double uy, double
 // ============================================================================
 // Gather of the post-stream populations of one site (zeroDown -> stream ->
 // wall rule -> periodic, coreLB.hpp:1319-1321, 814-818, in gather form).
-// For FP32 deviation storage the bookkeeping of the w*rho0 offsets is done in
-// FP64: base_j = (# of w-weighted contributions) - w_j.
+//
+// The small FP64 lattices are bound by the latency of dependent loads, so a
+// site's loads are issued in one round after its link word: the eight sources
+// (a slot that nothing streams into reads the site's own element), and, for a
+// site with wall links, its own populations and its type's specular targets
+// (one word per type).  Loading each wall link's population where the rule
+// uses it put up to eight round trips in a row: 5.9 us per 64 x 64 pass.
 // ============================================================================
-template <class S, int WALL>
-__device__ __forceinline__ void gather(const S* __restrict__ A, const Lat& L, int x, int y, int64_t p, uint32_t w,
-                                       const CellParam& ep, double rho0, double* f) {
+template <int WALL>
+__device__ __forceinline__ void gather(const double* __restrict__ A, const Lat& L, int x, int y, int64_t p, uint32_t w,
+                                       const CellParam& ep, double* f) {
 #pragma clang fp contract(off)
-    // rest population and streamed/periodic slots
-    f[0] = (double)Store<S>::ld(A, p);
-    double base[9];
-    base[0] = 0.0;
+    const uint32_t in = (w >> IN_SHIFT) & 0xffu, wall = (w >> WALL_SHIFT) & 0xffu;
+    double v[9], own[9];
+    uint32_t spec = 0;
+    v[0] = ld64(A, p);
 #pragma unroll
     for (int j = 1; j < 9; j++) {
-        const bool in = (w >> (IN_SHIFT + j - 1)) & 1u;
-        f[j] = in ? (double)Store<S>::ld(A, (int64_t)j * L.stride + L.src(x, y, j)) : 0.0;
-        base[j] = in ? 0.0 : -wq(j);
+        const int64_t s = L.src(x, y, j);
+        v[j] = ld64(A, (int64_t)j * L.stride + (((in >> (j - 1)) & 1u) ? s : p));
     }
-    const uint32_t wall = (w >> WALL_SHIFT) & 0xffu;
     if (wall) {
-        double keep[9];
 #pragma unroll
-        for (int j = 1; j < 9; j++) keep[j] = f[j];
-        const int t = (int)((w >> TYPE_SHIFT) & 63u);
+        for (int j = 1; j < 9; j++) own[j] = ld64(A, (int64_t)j * L.stride + p);
+        if (WALL != MTS_WALL_BB) spec = c_icsr4[(w >> TYPE_SHIFT) & 63u];
+    } else {
+#pragma unroll
+        for (int j = 1; j < 9; j++) own[j] = 0.0;
+    }
+    f[0] = v[0];
+#pragma unroll
+    for (int j = 1; j < 9; j++) {
+        v[j] = ((in >> (j - 1)) & 1u) ? v[j] : 0.0;
+        f[j] = v[j];
+    }
+    if (wall) {
         const double r = WALL == MTS_WALL_SRBB ? ep.r_srbb : 0.0;
 #pragma unroll
         for (int ic = 1; ic < 9; ic++) {
             if (!((wall >> (ic - 1)) & 1u)) continue;
-            const double a = (double)Store<S>::ld(A, (int64_t)ic * L.stride + p);
+            const double a = own[ic];
             if (WALL == MTS_WALL_BB) {
                 f[opp(ic)] = a;  // coreLB.hpp:859-865
-                base[opp(ic)] = wq(ic) - wq(opp(ic));
             } else {  // SRBB, coreLB.hpp:918-933
                 f[opp(ic)] += r * a;
-                base[opp(ic)] += r * wq(ic);
-                const int sr = c_icsr[t][ic];
+                const int sr = (int)((spec >> (4 * (ic - 1))) & 15u);
+                const double b = (1 - r) * a;
 #pragma unroll
                 for (int j = 1; j < 9; j++)
-                    if (sr == j) {
-                        f[j] += (1 - r) * a;
-                        base[j] += (1 - r) * wq(ic);
-                    }
+                    if (sr == j) f[j] += b;
             }
         }
         // periodic links overwrite after the wall rule (coreLB.hpp:969-977)
         if (w & SEAM_BIT) {
 #pragma unroll
             for (int j = 1; j < 9; j++)
-                if (L.seam_in(x, y, j) && ((w >> (IN_SHIFT + j - 1)) & 1u)) {
-                    f[j] = keep[j];
-                    base[j] = 0.0;
-                }
+                if (L.seam_in(x, y, j) && ((w >> (IN_SHIFT + j - 1)) & 1u)) f[j] = v[j];
         }
-    }
-    if (Store<S>::dev) {
-        // f currently holds sums of deviations; add back the offsets.
-#pragma unroll
-        for (int j = 0; j < 9; j++) f[j] = f[j] + wq(j) * rho0 + base[j] * rho0;
     }
 }
 
@@ -325,21 +319,22 @@ struct TransportArgs {
     const double *min_rho, *min_ux, *min_uy, *min_usq;
 };
 
-template <class S, int MODE, int COLL, int WALL>
+template <int MODE, int COLL, int WALL>
 __global__ void __launch_bounds__(256) k_transport(TransportArgs a) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y;
     if (x >= a.L.nx) return;
     const int64_t p = (int64_t)y * a.L.nx + x;
     const uint32_t w = a.meta[p];
+    const uint16_t pi = a.pidx[p];  // with the link word: one round trip
     if (!(w & FLUID_BIT)) return;
-    const CellParam ep = a.params[a.pidx[p]];
+    const CellParam ep = a.params[pi];
     double f[9];
     if (MODE == 0) {
 #pragma unroll
         for (int j = 0; j < 9; j++) f[j] = a.fcan[(int64_t)j * a.L.stride + p];
     } else {
-        gather<S, WALL>((const S*)a.Ain, a.L, x, y, p, w, ep, a.rho0, f);
+        gather<WALL>((const double*)a.Ain, a.L, x, y, p, w, ep, f);
     }
     if (MODE == 2) {
 #pragma unroll
@@ -358,21 +353,26 @@ __global__ void __launch_bounds__(256) k_transport(TransportArgs a) {
     else m = moments64(f, a.Fbody, a.fscale);
     if (a.usq_old) a.usq_old[p] = m.usq;
     collide64<COLL>(f, m, ep);
-    S* out = (S*)a.Aout;
+    double* out = (double*)a.Aout;
 #pragma unroll
-    for (int j = 0; j < 9; j++) {
-        const double v = Store<S>::dev ? f[j] - wq(j) * a.rho0 : f[j];
-        Store<S>::st(out, (int64_t)j * a.L.stride + p, (S)v);
-    }
+    for (int j = 0; j < 9; j++) st64(out, (int64_t)j * a.L.stride + p, f[j]);
 }
 
 // ============================================================================
-// Shan-Chen step (adsorption / coupled): LDS tile of TW x TH sites with a
-// one-site halo of FP64 pseudopotential.  MODE 0 collide-only from canonical
-// f, 1 fused.  The moments of the site (rho, u with the force shift), psi and
-// F can be written for output.
+// Shan-Chen step (adsorption / coupled): one thread per site of an SW x SH
+// region, the (SW - 2) x (SH - 2) tile in its middle and the ring of sites
+// around it.  Each thread gathers its site once, psi goes to LDS, and the
+// tile's threads finish from the populations they hold.  MODE 0 collide-only
+// from canonical f, 1 fused.  The moments of the site (rho, u with the force
+// shift), psi and F can be written for output.
+//
+// Bound: the latency of one wave's chain (link word, gather, psi, forces,
+// collision in FP64).  A 16 x 16 region recomputes psi for 1.31x the sites
+// and gives a 100 x 100 lattice 64 blocks; the former 64 x 16 tile with four
+// sites per thread gathered every site twice, one after the other, in 14
+// blocks.
 // ============================================================================
-constexpr int TW = 64, TH = 16, TROWS = 4;  // 256 threads = 64 x 4, 4 rows each
+constexpr int SW = 16, SH = 16;
 
 struct ScArgs {
     const void* Ain;
@@ -398,7 +398,7 @@ __device__ __forceinline__ double pseudo_potential(double rho, const ScArgs& a, 
     return neg ? acc : sqrt(acc);
 }
 
-template <class S, int MODE, int COLL, int WALL, bool GENPER>
+template <int MODE, int WALL, bool GENPER>
 __device__ __forceinline__ void site_f(const ScArgs& a, int x, int y, int64_t p, uint32_t w, const CellParam& ep,
                                        int64_t gpIn, int64_t gpOut, double rhoin, double* f) {
 #pragma clang fp contract(off)
@@ -406,7 +406,7 @@ __device__ __forceinline__ void site_f(const ScArgs& a, int x, int y, int64_t p,
 #pragma unroll
         for (int j = 0; j < 9; j++) f[j] = a.fcan[(int64_t)j * a.L.stride + p];
     } else {
-        gather<S, WALL>((const S*)a.Ain, a.L, x, y, p, w, ep, a.rho0, f);
+        gather<WALL>((const double*)a.Ain, a.L, x, y, p, w, ep, f);
         if (GENPER) {  // coreLB.hpp:980-1009 (W[2] on the diagonals)
             if (p == gpIn) {
                 f[1] = (1.0 / 9.0) * rhoin;
@@ -421,111 +421,92 @@ __device__ __forceinline__ void site_f(const ScArgs& a, int x, int y, int64_t p,
     }
 }
 
-template <class S, int MODE, int COLL, int WALL, bool GENPER>
-__global__ void __launch_bounds__(256) k_shanchen(ScArgs a, int64_t gpIn, int64_t gpOut, double rhoin) {
+template <int MODE, int COLL, int WALL, bool GENPER>
+__global__ void __launch_bounds__(SW * SH) k_shanchen(ScArgs a, int64_t gpIn, int64_t gpOut, double rhoin) {
 #pragma clang fp contract(off)
-    __shared__ double s_psi[TH + 2][TW + 2];
-    const int x0 = blockIdx.x * TW, y0 = blockIdx.y * TH;
-    const int tid = threadIdx.y * TW + threadIdx.x;
-    int neg = 0;
-    // phase 1: psi of the tile and its halo
-    for (int e = tid; e < (TH + 2) * (TW + 2); e += 256) {
-        const int hy = e / (TW + 2), hx = e % (TW + 2);
-        int gx = x0 - 1 + hx, gy = y0 - 1 + hy;
-        gx = gx < 0 ? gx + a.L.nx : (gx >= a.L.nx ? gx - a.L.nx : gx);
-        gy = gy < 0 ? gy + a.L.ny : (gy >= a.L.ny ? gy - a.L.ny : gy);
-        double ps = 0.0;
-        const bool inside = (x0 - 1 + hx) < a.L.nx + 1 && (y0 - 1 + hy) < a.L.ny + 1;
-        if (inside) {
-            const int64_t p = (int64_t)gy * a.L.nx + gx;
-            const uint32_t w = a.meta[p];
-            if (w & FLUID_BIT) {
-                const CellParam ep = a.params[a.pidx[p]];
-                double f[9];
-                site_f<S, MODE, COLL, WALL, GENPER>(a, gx, gy, p, w, ep, gpIn, gpOut, rhoin, f);
-                double r = 0.0;
+    __shared__ double s_psi[SH][SW];
+    const int hx = threadIdx.x % SW, hy = threadIdx.x / SW;
+    // the region's site, wrapped into the lattice; past the lattice's far edge
+    // only the first column and row (the wrapped neighbours) are used
+    const int ux_ = (int)blockIdx.x * (SW - 2) - 1 + hx, uy_ = (int)blockIdx.y * (SH - 2) - 1 + hy;
+    const bool inside = ux_ <= a.L.nx && uy_ <= a.L.ny;
+    const int x = ux_ < 0 ? ux_ + a.L.nx : (ux_ >= a.L.nx ? ux_ - a.L.nx : ux_);
+    const int y = uy_ < 0 ? uy_ + a.L.ny : (uy_ >= a.L.ny ? uy_ - a.L.ny : uy_);
+    const bool own = hx >= 1 && hx < SW - 1 && hy >= 1 && hy < SH - 1 && ux_ < a.L.nx && uy_ < a.L.ny;
+    int64_t p = 0;
+    uint32_t w = 0;
+    CellParam ep{};
+    double f[9], r = 0.0, ps = 0.0;
+    if (inside) {
+        p = (int64_t)y * a.L.nx + x;
+        w = a.meta[p];
+        const uint16_t pi = a.pidx[p];
+        if (w & FLUID_BIT) {
+            ep = a.params[pi];
+            site_f<MODE, WALL, GENPER>(a, x, y, p, w, ep, gpIn, gpOut, rhoin, f);
 #pragma unroll
-                for (int j = 0; j < 9; j++) r += f[j];
-                bool ng;
-                ps = pseudo_potential(r, a, ng);
-                const bool own = hx >= 1 && hx <= TW && hy >= 1 && hy <= TH;
-                if (own && ng) neg++;
-            }
+            for (int j = 0; j < 9; j++) r += f[j];
+            bool ng;
+            ps = pseudo_potential(r, a, ng);
+            if (a.psi_negative && own && ng) atomicAdd(a.psi_negative, 1);
         }
-        s_psi[hy][hx] = ps;
     }
+    s_psi[hy][hx] = ps;
     __syncthreads();
-    // phase 2: forces, velocity, collision, source for the tile's own sites
-    for (int k = 0; k < TROWS; k++) {
-        const int lx = threadIdx.x, ly = threadIdx.y + 4 * k;
-        const int x = x0 + lx, y = y0 + ly;
-        if (x >= a.L.nx || y >= a.L.ny) continue;
-        const int64_t p = (int64_t)y * a.L.nx + x;
-        const uint32_t w = a.meta[p];
-        if (!(w & FLUID_BIT)) continue;
-        const CellParam ep = a.params[a.pidx[p]];
-        double f[9];
-        site_f<S, MODE, COLL, WALL, GENPER>(a, x, y, p, w, ep, gpIn, gpOut, rhoin, f);
-        double r = 0.0, jx = 0.0, jy = 0.0;
+    if (!own || !(w & FLUID_BIT)) return;
+    double jx = 0.0, jy = 0.0;
 #pragma unroll
-        for (int j = 0; j < 9; j++) {
-            r += f[j];
-            if (ex(j) == 1) jx += f[j];
-            if (ex(j) == -1) jx += -f[j];
-            if (ey(j) == 1) jy += f[j];
-            if (ey(j) == -1) jy += -f[j];
-        }
-        // forces, coreLB.hpp:533-566
-        const double psi_i = s_psi[ly + 1][lx + 1];
-        double fxff = 0.0, fyff = 0.0, fxfw = 0.0, fyfw = 0.0;
-        const uint32_t outm = (w >> OUT_SHIFT) & 0xffu, wallm = (w >> WALL_SHIFT) & 0xffu;
+    for (int j = 0; j < 9; j++) {
+        if (ex(j) == 1) jx += f[j];
+        if (ex(j) == -1) jx += -f[j];
+        if (ey(j) == 1) jy += f[j];
+        if (ey(j) == -1) jy += -f[j];
+    }
+    // forces, coreLB.hpp:533-566
+    double fxff = 0.0, fyff = 0.0, fxfw = 0.0, fyfw = 0.0;
+    const uint32_t outm = (w >> OUT_SHIFT) & 0xffu, wallm = (w >> WALL_SHIFT) & 0xffu;
 #pragma unroll
-        for (int ic = 1; ic < 9; ic++) {
-            if ((outm >> (ic - 1)) & 1u) {
-                const double pn = s_psi[ly + 1 + ey(ic)][lx + 1 + ex(ic)];
-                const double c = (-6.0) * a.Gff * psi_i * wf(ic) * pn;
-                if (ex(ic) != 0) fxff += c * ex(ic);
-                if (ey(ic) != 0) fyff += c * ey(ic);
-            }
-            if ((wallm >> (ic - 1)) & 1u) {
-                const double c = (-1.0) * a.Gfs * psi_i * psi_i * wf(ic);
-                if (ex(ic) != 0) fxfw += c * ex(ic);
-                if (ey(ic) != 0) fyfw += c * ey(ic);
-            }
+    for (int ic = 1; ic < 9; ic++) {
+        if ((outm >> (ic - 1)) & 1u) {
+            const double pn = s_psi[hy + ey(ic)][hx + ex(ic)];
+            const double c = (-6.0) * a.Gff * ps * wf(ic) * pn;
+            if (ex(ic) != 0) fxff += c * ex(ic);
+            if (ey(ic) != 0) fyff += c * ey(ic);
         }
-        const double Fx = fxff + fxfw + a.Fbody, Fy = fyff + fyfw;
-        // velocity with the half-force shift, coreLB.hpp:1069-1099
-        Macro64 m;
-        m.rho = r;
-        m.ux = jx / r + Fx / (2.0 * r) * 1.0;
-        m.uy = jy / r + Fy / (2.0 * r) * 1.0;
-        m.usq = m.ux * m.ux + m.uy * m.uy;
-        if (a.rho) {
-            a.rho[p] = m.rho;
-            a.ux[p] = m.ux;
-            a.uy[p] = m.uy;
-            a.usq[p] = m.usq;
-        }
-        if (a.psi) {
-            a.psi[p] = psi_i;
-            a.Fx[p] = Fx;
-            a.Fy[p] = Fy;
-        }
-        collide64<COLL>(f, m, ep);
-        source64<COLL>(f, m.ux, m.uy, Fx, Fy, ep);
-        S* out = (S*)a.Aout;
-#pragma unroll
-        for (int j = 0; j < 9; j++) {
-            const double v = Store<S>::dev ? f[j] - wq(j) * a.rho0 : f[j];
-            Store<S>::st(out, (int64_t)j * a.L.stride + p, (S)v);
+        if ((wallm >> (ic - 1)) & 1u) {
+            const double c = (-1.0) * a.Gfs * ps * ps * wf(ic);
+            if (ex(ic) != 0) fxfw += c * ex(ic);
+            if (ey(ic) != 0) fyfw += c * ey(ic);
         }
     }
-    if (a.psi_negative && neg) atomicAdd(a.psi_negative, neg);
+    const double Fx = fxff + fxfw + a.Fbody, Fy = fyff + fyfw;
+    // velocity with the half-force shift, coreLB.hpp:1069-1099
+    Macro64 m;
+    m.rho = r;
+    m.ux = jx / r + Fx / (2.0 * r) * 1.0;
+    m.uy = jy / r + Fy / (2.0 * r) * 1.0;
+    m.usq = m.ux * m.ux + m.uy * m.uy;
+    if (a.rho) {
+        a.rho[p] = m.rho;
+        a.ux[p] = m.ux;
+        a.uy[p] = m.uy;
+        a.usq[p] = m.usq;
+    }
+    if (a.psi) {
+        a.psi[p] = ps;
+        a.Fx[p] = Fx;
+        a.Fy[p] = Fy;
+    }
+    collide64<COLL>(f, m, ep);
+    source64<COLL>(f, m.ux, m.uy, Fx, Fy, ep);
+    double* out = (double*)a.Aout;
+#pragma unroll
+    for (int j = 0; j < 9; j++) st64(out, (int64_t)j * a.L.stride + p, f[j]);
 }
 
 // Stream-only pass of the Shan-Chen steps: A -> canonical f (wall rule of the
 // step, periodic, generalized periodic).
-template <class S, int WALL, bool GENPER>
+template <int WALL, bool GENPER>
 __global__ void __launch_bounds__(256) k_sc_stream(ScArgs a, int64_t gpIn, int64_t gpOut, double rhoin) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y;
@@ -535,7 +516,7 @@ __global__ void __launch_bounds__(256) k_sc_stream(ScArgs a, int64_t gpIn, int64
     if (!(w & FLUID_BIT)) return;
     const CellParam ep = a.params[a.pidx[p]];
     double f[9];
-    site_f<S, 1, MTS_COLL_MRT, WALL, GENPER>(a, x, y, p, w, ep, gpIn, gpOut, rhoin, f);
+    site_f<1, WALL, GENPER>(a, x, y, p, w, ep, gpIn, gpOut, rhoin, f);
     double* fc = const_cast<double*>(a.fcan);
 #pragma unroll
     for (int j = 0; j < 9; j++) fc[(int64_t)j * a.L.stride + p] = f[j];
@@ -701,20 +682,26 @@ void upload_icsr(hipStream_t st) {
     for (int i = 0; i < MTS_NTYPES; i++)
         for (int j = 0; j < 9; j++) t[i][j] = MTS_ICSR[i][j] < 0 ? 0 : MTS_ICSR[i][j];
     for (int j = 0; j < 9; j++) t[MTS_NTYPES][j] = (signed char)OPP[j];
+    static uint32_t t4[64];
+    for (int i = 0; i < 64; i++) {
+        t4[i] = 0;
+        for (int j = 1; j < 9; j++) t4[i] |= (uint32_t)t[i < MTS_NTYPES ? i : MTS_NTYPES][j] << (4 * (j - 1));
+    }
+    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_icsr4), t4, sizeof(t4), 0, hipMemcpyHostToDevice, st);
     (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_icsr), t, sizeof(t), 0, hipMemcpyHostToDevice, st);
 }
 
-template <class S, int MODE, int COLL, int WALL>
+template <int MODE, int COLL, int WALL>
 static void launch_t(const LaunchCtx& c, const TransportArgs& a) {
     dim3 blk(256, 1), grd((c.nx + 255) / 256, c.ny);
-    klaunch(k_transport<S, MODE, COLL, WALL>, grd, blk, 0, c, a);
+    klaunch(k_transport<MODE, COLL, WALL>, grd, blk, 0, c, a);
 }
 
-template <class S, int MODE>
+template <int MODE>
 static int dispatch_t(const LaunchCtx& c, const TransportArgs& a, int coll, int wall) {
 #define MTS_T(CO, WA)                                      \
     if (coll == CO && wall == WA) {                        \
-        launch_t<S, MODE, CO, WA>(c, a);                   \
+        launch_t<MODE, CO, WA>(c, a);                   \
         return 0;                                          \
     }
     MTS_T(MTS_COLL_RMRT, MTS_WALL_SRBB)
@@ -749,33 +736,32 @@ int launch_transport(const LaunchCtx& c, int mode, const TransportSpec& s) {
     a.min_uy = s.min_uy;
     a.min_usq = s.min_usq;
     if (c.fp32) return c.cimg ? launch_ctransport(c, mode, s) : MTS_ERR_STATE;  // FP32 runs in cell order
-    if (mode == 0) return dispatch_t<double, 0>(c, a, c.coll, c.wall);
-    if (mode == 1) return dispatch_t<double, 1>(c, a, c.coll, c.wall);
-    return dispatch_t<double, 2>(c, a, c.coll, c.wall);
+    if (mode == 0) return dispatch_t<0>(c, a, c.coll, c.wall);
+    if (mode == 1) return dispatch_t<1>(c, a, c.coll, c.wall);
+    return dispatch_t<2>(c, a, c.coll, c.wall);
 }
 
-template <class S, int MODE, int COLL, int WALL, bool GP>
+template <int MODE, int COLL, int WALL, bool GP>
 static void launch_sc(const LaunchCtx& c, const ScArgs& a) {
-    dim3 blk(TW, 4), grd((c.nx + TW - 1) / TW, (c.ny + TH - 1) / TH);
-    hipLaunchKernelGGL((k_shanchen<S, MODE, COLL, WALL, GP>), grd, blk, 0, c.stream, a, c.gpIn, c.gpOut, c.rhoin);
+    dim3 blk(SW * SH), grd((c.nx + SW - 3) / (SW - 2), (c.ny + SH - 3) / (SH - 2));
+    hipLaunchKernelGGL((k_shanchen<MODE, COLL, WALL, GP>), grd, blk, 0, c.stream, a, c.gpIn, c.gpOut, c.rhoin);
 }
-template <class S, int WALL, bool GP>
+template <int WALL, bool GP>
 static void launch_scs(const LaunchCtx& c, const ScArgs& a) {
     dim3 blk(256, 1), grd((c.nx + 255) / 256, c.ny);
-    hipLaunchKernelGGL((k_sc_stream<S, WALL, GP>), grd, blk, 0, c.stream, a, c.gpIn, c.gpOut, c.rhoin);
+    hipLaunchKernelGGL((k_sc_stream<WALL, GP>), grd, blk, 0, c.stream, a, c.gpIn, c.gpOut, c.rhoin);
 }
 
 // kind 0 adsorption (MRT, BB, generalized periodic); kind 1 coupled (RMRT, SRBB)
-template <class S>
 static void sc_dispatch(const LaunchCtx& c, int kind, int mode, const ScArgs& a) {
     if (kind == 0) {
-        if (mode == 0) launch_sc<S, 0, MTS_COLL_MRT, MTS_WALL_BB, true>(c, a);
-        else if (mode == 1) launch_sc<S, 1, MTS_COLL_MRT, MTS_WALL_BB, true>(c, a);
-        else launch_scs<S, MTS_WALL_BB, true>(c, a);
+        if (mode == 0) launch_sc<0, MTS_COLL_MRT, MTS_WALL_BB, true>(c, a);
+        else if (mode == 1) launch_sc<1, MTS_COLL_MRT, MTS_WALL_BB, true>(c, a);
+        else launch_scs<MTS_WALL_BB, true>(c, a);
     } else {
-        if (mode == 0) launch_sc<S, 0, MTS_COLL_RMRT, MTS_WALL_SRBB, false>(c, a);
-        else if (mode == 1) launch_sc<S, 1, MTS_COLL_RMRT, MTS_WALL_SRBB, false>(c, a);
-        else launch_scs<S, MTS_WALL_SRBB, false>(c, a);
+        if (mode == 0) launch_sc<0, MTS_COLL_RMRT, MTS_WALL_SRBB, false>(c, a);
+        else if (mode == 1) launch_sc<1, MTS_COLL_RMRT, MTS_WALL_SRBB, false>(c, a);
+        else launch_scs<MTS_WALL_SRBB, false>(c, a);
     }
 }
 
@@ -804,7 +790,7 @@ int launch_shanchen(const LaunchCtx& c, int kind, int mode, const ScSpec& s) {
     a.Fy = s.Fy;
     a.psi_negative = s.psi_negative;
     if (c.fp32) return c.cimg ? launch_cshanchen(c, kind, mode, s) : MTS_ERR_STATE;
-    sc_dispatch<double>(c, kind, mode, a);
+    sc_dispatch(c, kind, mode, a);
     return 0;
 }
 
