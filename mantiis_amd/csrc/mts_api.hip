@@ -320,6 +320,7 @@ static int upload_compact(mts_sim_s* s, const CompactImage& h, const float* cpar
     d.book = s->d_book;
     d.ncell = h.ncell;
     d.cstride = h.cstride;
+    d.inplace = compact_inplace(h);
     d.ntx = h.ntx;
     return MTS_OK;
 }
@@ -657,7 +658,7 @@ static int create_multi32(mts_sim_s* s, const std::vector<CoarseRow>& cr, const 
         build_compact(v, C.h);
         if ((rc = upload_compact(s, C.h, cpar, C.plain))) return rc;
         const int64_t OS = std::max<int64_t>((nslot + 63) / 64 * 64, 64);
-        if ((rc = s->alloc(&C.A[0], (size_t)C.h.cstride * 9)) || (rc = s->alloc(&C.A[1], (size_t)C.h.cstride * 9)) ||
+        if ((rc = s->alloc(&C.A[0], (size_t)C.h.cstride * 9 + PLANE_GUARD)) || (rc = s->alloc(&C.A[1], (size_t)C.h.cstride * 9 + PLANE_GUARD)) ||
             (rc = s->alloc(&C.m[0], (size_t)C.h.cstride * 3)) || (rc = s->alloc(&C.m[1], (size_t)C.h.cstride * 3)) ||
             (rc = s->alloc(&C.O, (size_t)OS * 9)))
             return rc;
@@ -1189,7 +1190,7 @@ int mts_create(int nx, int ny, const int32_t* pore, const double* kn, const doub
     const size_t np = (size_t)g.stride * 9;
     const bool fp32 = prm.precision == MTS_FP32DEV;
     if (fp32) build_compact(g, s->cimg_h);
-    const size_t nA = fp32 ? (size_t)s->cimg_h.cstride * 9 * 4 : np * 8;
+    const size_t nA = fp32 ? ((size_t)s->cimg_h.cstride * 9 + PLANE_GUARD) * 4 : np * 8;
     s->nparts = (int)std::min<int64_t>(1024, (s->P + 255) / 256);
     if ((rc = s->alloc(&s->d_meta, s->P)) || (rc = s->alloc(&s->d_pidx, s->P)) ||
         (rc = s->alloc(&s->d_params, g.params.size())) || (rc = s->alloc(&s->d_cellPos, g.ncell)) ||
@@ -1525,11 +1526,22 @@ int mts_step_transport(mts_sim s, int nsteps) {
     t.usq_old = nsteps == 1 ? s->d_usq_old : nullptr;
     t.Mout = s->d_M[0];
     if ((rc = launch_transport(c, 0, t))) return fail(rc, "operator combination has no fused kernel");
+    // fused passes: pairs in place where the FP32 image allows it (an odd
+    // count starts with a pass to the other copy)
+    const bool pairs = s->use_cimg && s->cimg.inplace && !mdbb;
     for (int i = 1; i < nsteps; i++) {
         TransportSpec u;
+        u.usq_old = (i == nsteps - 1) ? s->d_usq_old : nullptr;
+        const int left = nsteps - i;  // passes to go
+        if (pairs && !(i == 1 && (left & 1))) {
+            u.Aout = s->d_A;
+            s->tick(c);
+            launch_transport(c, left & 1 ? 4 : 3, u);
+            s->tock(c);
+            continue;
+        }
         u.Ain = s->d_A;
         u.Aout = s->d_B;
-        u.usq_old = (i == nsteps - 1) ? s->d_usq_old : nullptr;
         u.Min = s->d_M[mc];
         u.Mout = s->d_M[mc ^ 1];
         s->tick(c);

@@ -208,12 +208,24 @@ struct mts_batch_s {
             if (nsteps & 1) return advance(1, false);
             return MTS_OK;
         }
-        for (int i = 0; i < nsteps; i++)
-            if ((rc = step(false, 0))) return rc;
+        return plain(nsteps, false);
+    }
+    // nsteps one-step launches, the last with statistics if asked for.  Pairs
+    // run in place where the image allows it (an odd count starts with a step
+    // to the other buffer, so the buffer changes as often as without pairs,
+    // modulo two, and lattices outside the queue are where they were)
+    int plain(int nsteps, bool stats) {
+        int rc;
+        const bool pairs = dev.inplace && prm.wall != MTS_WALL_MDBB;
+        for (int i = 0; i < nsteps; i++) {
+            const bool last = i == nsteps - 1;
+            const int form = !pairs ? 0 : (nsteps & 1) ? (i == 0 ? 0 : 2 - (i & 1)) : 1 + (i & 1);
+            if ((rc = step(stats && last, 0, form))) return rc;
+        }
         return MTS_OK;
     }
-    // one step over the queue: A[cur] -> A[cur^1]
-    int step(bool stats, int from) {
+    // one step over the queue: A[cur] -> A[cur^1], or in place (form 1, 2)
+    int step(bool stats, int from, int form = 0) {
         BatchLaunch L;
         L.c = ctx();
         L.Ain = A[cur];
@@ -227,14 +239,17 @@ struct mts_batch_s {
         L.xrun = xrun;
         L.Min = M[cur];
         L.Mout = M[cur ^ 1];
+        L.raw = tiled;
         if (from == 2) {  // the given state sits in A[cur^1]: read it, write A[cur]
             L.Ain = A[cur ^ 1];
             L.Aout = A[cur];
             L.Mout = M[cur];
         }
+        L.form = form;
+        if (form) L.Aout = A[cur];
         const int rc = launch_cbatch(L);
         if (stats) launch_bsum(part, d_first, acc, nb, stream);
-        if (from != 2) cur ^= 1;
+        if (from != 2 && !form) cur ^= 1;
         return rc;
     }
     // n steps (n even), the last with statistics
@@ -245,9 +260,7 @@ struct mts_batch_s {
                 if ((rc = advance(2, i == n / 2 - 1))) return rc;
             return MTS_OK;
         }
-        for (int i = 0; i < n; i++)
-            if ((rc = step(i == n - 1, 0))) return rc;
-        return MTS_OK;
+        return plain(n, true);
     }
     // Autotuner: times every launch configuration (threads per block x XCD
     // run length) for `each` steps from the current state and keeps the
@@ -364,7 +377,7 @@ struct mts_batch_s {
             ggrid = grid_key();
         }
         BT_TRY(hipGraphLaunch(gexec, stream));
-        const int flips = tiled ? n / 2 : n;  // launches in the chunk
+        const int flips = tiled ? n / 2 : 0;  // n is even: plain steps end in the buffer they began in
         if (flips & 1) cur ^= 1;
         return MTS_OK;
     }
@@ -534,6 +547,7 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
             b->blocks_of[g].push_back(B.id);
             b->hblocks.push_back(B);
         }
+        C.nraw += ci.nraw;
         base += ((n + 255) / 256) * 256;
         // padding cells between lattices are never in a block
         C.cw.resize(base, 0);
@@ -563,7 +577,7 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
     float* cpar;
     std::vector<float> book;
     fp32_params(b->params, b->ph.rhoin, b->cpar_h, book);
-    const size_t nA = (size_t)base * 9;
+    const size_t nA = (size_t)base * 9 + PLANE_GUARD;
     if ((rc = b->alloc(&cw, base)) || (rc = b->alloc(&rw, base)) || (rc = b->alloc(&pidx, base)) ||
         (rc = b->alloc(&outm, base)) || (rc = b->alloc(&aux, std::max<size_t>(C.aux.size(), 1))) ||
         (rc = b->alloc(&cpar, b->cpar_h.size())) || (rc = b->alloc(&b->book, book.size())) ||
@@ -619,6 +633,7 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
     b->dev.book = b->book;
     b->dev.ncell = base;
     b->dev.cstride = base;
+    b->dev.inplace = !b->tiled && compact_inplace(C);
     // drop the host copies of what now lives on the device
     C.cw = std::vector<uint32_t>();
     C.rw = std::vector<uint32_t>();

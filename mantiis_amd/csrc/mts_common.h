@@ -96,16 +96,24 @@ int build_single_grid(int nx, int ny, const int32_t* pore, const double* kn, con
 //             the x neighbours of a cell are the cells c-1 and c+1;
 //   outm:     the OUT bits (Shan-Chen neighbour sum).
 // A COMPLEX cell (lattice columns 0 and nx-1, x-seam sites, the generalized-
-// periodic cells and cells whose wall links share a specular slot) keeps its
+// periodic cells, cells whose wall links share a specular slot and cells whose
+// wall-fed slots are not the opposites of their wall links) keeps its
 // sources, position and full link word in an aux record; its rw is the record.
 constexpr uint32_t CW_WALL_SHIFT = 8, CW_TYPE_SHIFT = 16;
 constexpr uint32_t CW_COMPLEX = 1u << 22, CW_ISC_D = 1u << 23, CW_ISC_U = 1u << 24;
 constexpr uint32_t CW_X_SHIFT = 25;
+// A COMPLEX cell has no rank bits; bit 23 marks it RAW: its wall rule is applied
+// in link order when it is gathered (x-seam sites, buffer cells, irregular
+// wall links).  The others only take their sources from the record.
+constexpr uint32_t CW_RAW = CW_COMPLEX | CW_ISC_D;
 constexpr int CTILE_W = 128, CTILE_H = 8;  // Shan-Chen tile (sites)
+constexpr int CPAR_FLOATS = 12;  // FP32 parameter record of one (tau_s, Kn) pair
+constexpr int PLANE_GUARD = 64;  // elements after the last population plane (a neighbour index may be the cell count)
 constexpr int AUXW = 12;  // aux record: src[8], x, y, link word, override slot (-1: none)
 
 struct CompactImage {
     int64_t ncell = 0, cstride = 0, naux = 0;
+    int64_t nraw = 0;              // RAW cells
     int ntx = 0;                   // tile columns of CTILE_W sites
     std::vector<uint32_t> cw;      // [ncell]
     std::vector<uint32_t> rw;      // [ncell]: packed rank offsets (COMPLEX: aux record)
@@ -135,6 +143,12 @@ struct LatticeView {
     int64_t gpIn, gpOut;
     const int32_t* override;
 };
+
+// Whether steps may write where they read: no RAW cell, and every element of
+// the nine planes within reach of a 32-bit byte offset.
+inline bool compact_inplace(const CompactImage& ci) {
+    return ci.nraw == 0 && ((uint64_t)ci.cstride * 9 + PLANE_GUARD) * 4 < ((uint64_t)1 << 32);
+}
 
 // Builds the cell-order image of a single-block lattice or of one level.
 void build_compact(const Geometry& g, CompactImage& ci);

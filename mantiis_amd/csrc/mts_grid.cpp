@@ -309,6 +309,7 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
     ci.pidx.assign(n, 0);
     ci.outm.assign(n, 0);
     ci.aux.clear();
+    ci.nraw = 0;
     canonical_spec(ci.spec);
     for (int64_t c = 0; c < n; c++) {
         const int64_t p = ci.cellPos[c];
@@ -332,16 +333,21 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
             if ((spec >> (4 * (sr - 1))) & 15u) ambiguous = true;
             spec |= (uint32_t)ic << (4 * (sr - 1));
         }
-        // rows 0 and ny-1 of a non-torus lattice lose their y-seam links
-        // the kernel takes slot j's specular source from the type table,
-        // kept when that source is one of the cell's wall links
-        uint32_t specT = 0;
+        // A simple cell's slot j streams or is fed by its wall rule, and then
+        // population opp(j) reaches no other cell: its plane holds the fed
+        // value between passes.  Its specular sources are those of its type
+        // (the kernels' table).  Cells that break this are RAW.
+        bool irregular = wall != 0 && spec != ci.spec[t];
         for (int j = 1; j < 9; j++) {
-            const uint32_t sj = (ci.spec[t] >> (4 * (j - 1))) & 15u;
-            if (sj && ((wall >> (sj - 1)) & 1u)) specT |= sj << (4 * (j - 1));
+            const bool inj = (in >> (j - 1)) & 1u, fed = (wall >> (OPP[j] - 1)) & 1u;
+            if (inj == fed || (inj && ((spec >> (4 * (j - 1))) & 15u))) irregular = true;
+            if (!((wall >> (j - 1)) & 1u)) continue;
+            const int64_t q = (int64_t)wrap(y + EY[j], ny) * nx + wrap(x + EX[j], nx);
+            if (ci.cidx[q] >= 0 && ((g.meta[q] >> (IN_SHIFT + j - 1)) & 1u)) irregular = true;
         }
-        const bool complex = (w & SEAM_BIT) || x == 0 || x == nx - 1 || (!g.torus && (y == 0 || y == ny - 1)) ||
-                             ambiguous || specT != spec || p == g.gpIn || p == g.gpOut || ny < 3 || ovr >= 0;
+        const bool raw = irregular || (w & SEAM_BIT) || ambiguous || ovr >= 0;
+        const bool complex = raw || x == 0 || x == nx - 1 || (!g.torus && (y == 0 || y == ny - 1)) ||  // y-seam links lost
+                             p == g.gpIn || p == g.gpOut || ny < 3;
         auto push_aux = [&]() {  // explicit record of a COMPLEX cell
             const int32_t k = (int32_t)(ci.aux.size() / AUXW);
             for (int j = 1; j < 9; j++) {
@@ -362,7 +368,8 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
         const int64_t du = (int64_t)rank[pu] - c, dd = c - (int64_t)rank[pd];
         const bool fits = du >= -32768 && du <= 32767 && dd >= -32768 && dd <= 32767;
         if (complex || !fits) {
-            cw |= CW_COMPLEX;
+            cw = (cw & ~(CW_ISC_D | CW_ISC_U)) | (raw ? CW_RAW : CW_COMPLEX);
+            ci.nraw += raw;
             ci.rw[c] = (uint32_t)push_aux();
         } else {
             ci.rw[c] = ((uint32_t)(uint16_t)(int16_t)du) | ((uint32_t)(uint16_t)(int16_t)dd << 16);
@@ -377,7 +384,7 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
                 if (ci.cidx[(int64_t)ys * nx + xs] != src[j]) ok = false;
             }
             if (!ok) {
-                cw |= CW_COMPLEX;
+                cw = (cw & ~(CW_ISC_D | CW_ISC_U)) | CW_COMPLEX;
                 ci.rw[c] = (uint32_t)push_aux();
             }
         }

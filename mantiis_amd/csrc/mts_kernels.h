@@ -18,7 +18,7 @@ struct CompactDev {
     const int32_t* aux = nullptr;
     const int32_t* cidx = nullptr;
     const int32_t* segs = nullptr;
-    const void* cpar = nullptr;  // FP32 parameter records (32 B per (tau_s, Kn) pair)
+    const void* cpar = nullptr;  // FP32 parameter records (CPAR_FLOATS per (tau_s, Kn) pair)
     const void* book = nullptr;  // SRBB bookkeeping table (24 floats per pair)
     const int32_t* cellPos = nullptr;
     int64_t ncell = 0, cstride = 0;
@@ -27,6 +27,7 @@ struct CompactDev {
     int64_t OS = 0;
     int ovr = 0;  // 0 gather, 1 take the override, 2 skip (see CImg)
     const float* M = nullptr;  // MDBB state read by the gather (set per launch)
+    bool inplace = false;      // steps may write where they read (no RAW cell, planes within 4 GiB)
 };
 
 struct LaunchCtx {
@@ -189,6 +190,8 @@ struct BatchLaunch {
     int xrun = 32;           // XCD run length of the queue map (0: none)
     const float* Min = nullptr;  // MDBB state (see TransportSpec)
     float* Mout = nullptr;
+    int form = 0;      // 0: Ain -> Aout; 1, 2: the odd and the even step in place on Aout
+    bool raw = false;  // keep the populations of wall links (the tile kernels apply the wall rule themselves)
 };
 int launch_cbatch(const BatchLaunch& L);
 // Batched tile kernels (mts_tile.inc): one block per TILE_X x TILE_Y site

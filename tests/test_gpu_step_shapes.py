@@ -40,3 +40,35 @@ def test_shan_chen_fp64_tile_edges(n, kind, coll, wall):
     # same operations in the same order: FP64 rounding of 12 (112) steps
     for name in ("f", "rho", "ux", "uy"):
         assert rel_l2(g.get(name), o.get(name)) <= 1e-12, name
+
+
+# FP32 steps run in pairs that write where they read; odd counts start with a
+# pass to the other copy.  f deviates from w rho0 by what 16 roundings of 2^-24
+# per step can add up to (times 4: the sums of nine).
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("n,coll,wall,pairs", [(4, 2, 2, 1), (5, 2, 0, 1), (17, 0, 2, 2), (33, 1, 2, 1), (64, 2, 2, 3),
+                                               (65, 2, 2, 1), (100, 1, 0, 1)])
+def test_fp32_transport_in_place(n, coll, wall, pairs, steps):
+    banner(f"FP32 in-place transport {n} x {n}, collision {coll}, wall {wall}, {pairs} pairs, {steps} steps")
+    if n < 12:
+        pore = np.ones((n, n), np.int32)  # no wall: every slot streams over the seams
+    else:
+        pore = cut(n, 11)[0] if n <= 64 else G.disk_packing(n, 0.65, 3, 7, seed=5)
+    kn, lp = G.uniform_kn(pore, 0.1, MFP_DX)
+    for k in range(1, pairs):  # vertical bands of other Knudsen numbers
+        kn[:, k::pairs] *= 1 + 0.5 * k
+        lp[:, k::pairs] /= 1 + 0.5 * k
+    par = dict(dx=1e-9, Fbody=1e-6)
+    o = O.Oracle(pore, kn, lp, periodic_y=True, **par)
+    o.set_operators(coll, wall)
+    o.run("transport", steps, 0.0)
+    g = Lattice(pore, kn, lp, precision="fp32dev", collision=coll, wall=wall, periodic_y=1, **par)
+    g.step("transport", steps)
+    w = np.array([4 / 9] + [1 / 9] * 4 + [1 / 36] * 4)
+    rho0 = 0.235554544075989  # default gas state
+    a, b = (np.asarray(x.get("f")).reshape(-1, 9) - w * rho0 for x in (g, o))
+    assert rel_l2(a, b) <= 4 * 16 * 2.0**-24 * (steps + 1)
+    g.step("transport", steps)  # a second call goes on from the canonical state
+    o.run("transport", steps, 0.0)
+    a, b = (np.asarray(x.get("f")).reshape(-1, 9) - w * rho0 for x in (g, o))
+    assert rel_l2(a, b) <= 4 * 16 * 2.0**-24 * (2 * steps + 2)
