@@ -15,6 +15,7 @@
 #include "mantiis_hip.h"
 #include "mts_common.h"
 #include "mts_kernels.h"
+#include "mts_readback.h"
 #include "mts_multigrid.h"
 
 namespace mts {
@@ -57,6 +58,7 @@ struct mts_sim_s {
     mts_params prm{};
     hipStream_t stream = nullptr;
     int64_t P = 0;
+    Readback readback;
     uint32_t* d_meta = nullptr;
     uint16_t* d_pidx = nullptr;
     CellParam* d_params = nullptr;
@@ -99,6 +101,9 @@ struct mts_sim_s {
         double *d_ftemp = nullptr, *d_feq = nullptr, *d_fneq = nullptr, *d_fb = nullptr, *d_rho_old = nullptr;
     };
     bool multi = false;
+    // pixel -> covering non-buffer cell: its level (0: wall) and level-image site
+    uint8_t* d_pixLevel = nullptr;
+    int32_t* d_pixSite = nullptr;
     MultiGeometry mg;
     std::vector<LevelImage> limg;
     std::vector<LevelDev> lv;
@@ -804,6 +809,28 @@ static int create_multi(mts_sim_s* s, int nx, int ny, const int32_t* pore, const
         (rc = upload(s->d_frows, fr.data(), fr.size() * sizeof(FineRow), s->stream)))
         return rc;
     if (s->prm.precision == MTS_FP32DEV && (rc = create_multi32(s, cr, fr, err))) return rc;
+    {
+        const size_t np = (size_t)nx * ny;
+        std::vector<uint8_t> lev(np, 0);
+        std::vector<int32_t> site(np, 0);
+        for (int64_t c = 0; c < s->mg.ncell; c++) {
+            if (s->mg.isBuffer[c]) continue;
+            const int l = s->mg.level[c] - 1, w = 1 << l;
+            const int32_t q = (int32_t)((int64_t)(s->mg.cy[c] >> l) * s->lv[l].nx + (s->mg.cx[c] >> l));
+            for (int dy = 0; dy < w; dy++)
+                for (int dx = 0; dx < w; dx++) {
+                    const size_t p = (size_t)(s->mg.cy[c] + dy) * nx + s->mg.cx[c] + dx;
+                    lev[p] = (uint8_t)(l + 1);
+                    site[p] = q;
+                }
+        }
+        if ((rc = s->alloc(&s->d_pixLevel, np)) || (rc = s->alloc(&s->d_pixSite, np)) ||
+            (rc = upload(s->d_pixLevel, lev.data(), np, s->stream)) ||
+            (rc = upload(s->d_pixSite, site.data(), np * 4, s->stream)))
+            return rc;
+        HIP_TRY(hipStreamSynchronize(s->stream));  // the host maps go out of scope
+        if (np * 24 >= Readback::MIN_BYTES) (void)s->readback.ready();
+    }
     upload_icsr(s->stream);
     upload_xynorm(s->stream);
     for (size_t l = 0; l < s->lv.size(); l++) {
@@ -1217,6 +1244,7 @@ int mts_create(int nx, int ny, const int32_t* pore, const double* kn, const doub
     upload_icsr(s->stream);
     upload_xynorm(s->stream);
     *out = s;
+    if ((size_t)s->P * 24 >= Readback::MIN_BYTES) (void)s->readback.ready();
     rc = mts_initialize(s);
     if (rc) {
         *out = nullptr;
@@ -1906,40 +1934,30 @@ int mts_set_field(mts_sim s, int field, const double* in) {
 
 int mts_complete_domain(mts_sim s, double* ux, double* uy, double* rho) {
     if (!s) return fail(MTS_ERR_ARG, "null handle");
-    if (s->multi) {
-        // each pixel takes the value of the non-buffer cell covering it (the
-        // assignment of coreLB.hpp:1413-1552); wall pixels 0
-        const int nx = s->mg.nx, ny = s->mg.ny;
-        const int64_t n = s->mg.ncell;
-        std::vector<double> a(n), b(n), c(n);
-        int rc;
-        if ((rc = multi_get(s, MTS_F_UX, a.data())) || (rc = multi_get(s, MTS_F_UY, b.data())) ||
-            (rc = multi_get(s, MTS_F_RHO, c.data())))
-            return rc;
-        double* outs[3] = {ux, uy, rho};
-        const std::vector<double>* vals[3] = {&a, &b, &c};
-        for (int k = 0; k < 3; k++)
-            if (outs[k]) std::fill(outs[k], outs[k] + (size_t)nx * ny, 0.0);
-        for (int64_t cc = 0; cc < n; cc++) {
-            if (s->mg.isBuffer[cc]) continue;
-            const int w = 1 << (s->mg.level[cc] - 1);
-            for (int dy = 0; dy < w; dy++)
-                for (int dx = 0; dx < w; dx++) {
-                    const size_t p = (size_t)(s->mg.cy[cc] + dy) * nx + s->mg.cx[cc] + dx;
-                    for (int k = 0; k < 3; k++)
-                        if (outs[k]) outs[k][p] = (*vals[k])[cc];
-                }
-        }
-        return MTS_OK;
-    }
     double* outs[3] = {ux, uy, rho};
     double* src[3] = {s->d_ux, s->d_uy, s->d_rho};
-    for (int k = 0; k < 3; k++) {
-        if (!outs[k]) continue;
-        // dense site image is row-major and holds 0 at solid sites
-        HIP_TRY(hipMemcpyAsync(outs[k], src[k], s->P * 8, hipMemcpyDeviceToHost, s->stream));
+    int64_t P = s->P;
+    if (s->multi) {
+        // each pixel takes the value of the non-buffer cell covering it (the
+        // assignment of coreLB.hpp:1413-1552); wall pixels 0.  The pixel
+        // images are formed in the finest level's population buffer, which
+        // holds nothing between calls.
+        P = (int64_t)s->mg.nx * s->mg.ny;
+        PixelSpec px;
+        for (size_t l = 0; l < s->lv.size(); l++) {
+            px.ux[l] = s->lv[l].d_ux;
+            px.uy[l] = s->lv[l].d_uy;
+            px.rho[l] = s->lv[l].d_rho;
+        }
+        for (int k = 0; k < 3; k++) px.out[k] = src[k] = (double*)s->lv[0].d_A + k * P;
+        launch_pixel_out(s->stream, P, s->d_pixLevel, s->d_pixSite, px);
+        if (int rc = s->launched()) return rc;
     }
-    HIP_TRY(hipStreamSynchronize(s->stream));
+    // the dense site image is row-major and holds 0 at solid sites
+    std::vector<Readback::Piece> pieces;
+    for (int k = 0; k < 3; k++)
+        if (outs[k]) pieces.push_back({outs[k], src[k], (size_t)P * 8});
+    HIP_TRY(s->readback.run(s->prm.device, s->stream, pieces));
     return MTS_OK;
 }
 

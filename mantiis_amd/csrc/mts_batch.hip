@@ -18,6 +18,7 @@
 #include "mantiis_hip.h"
 #include "mts_common.h"
 #include "mts_kernels.h"
+#include "mts_readback.h"
 
 using namespace mts;
 
@@ -54,6 +55,7 @@ struct mts_batch_s {
     float* msnap = nullptr;
     int cur = 0;
     float* mac = nullptr;
+    Readback readback;
     double* acc = nullptr;
     double* part = nullptr;      // per block
     int32_t* d_first = nullptr;  // per lattice: first block id (nb + 1)
@@ -643,6 +645,7 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
     b->active.assign(nb, 1);
     b->u_prev.assign(nb, 0.0);
     if ((rc = b->upload_queue())) return bail(rc);
+    if (*std::max_element(b->ncell.begin(), b->ncell.end()) * 12 >= (int64_t)Readback::SLOT) (void)b->readback.ready();
     if ((rc = b->step(true, 1))) return bail(rc);  // rest equilibrium -> first post-collision state
     e = hipStreamSynchronize(b->stream);
     if (e == hipSuccess) e = hipGetLastError();
@@ -778,20 +781,51 @@ int mts_batch_fields(mts_batch b, int g, double* rho, double* ux, double* uy) {
     if (int rc = check(b)) return rc;
     if (g < 0 || g >= b->nb || !rho || !ux || !uy) return set_error(MTS_ERR_ARG, "bad argument");
     const int64_t n = b->ncell[g], o = b->off[g], S = b->dev.cstride;
-    std::vector<float> h(3 * n);
-    for (int k = 0; k < 3; k++)
-        BT_TRY(hipMemcpyAsync(&h[k * n], b->mac + k * S + o, n * 4, hipMemcpyDeviceToHost, b->stream));
-    BT_TRY(hipStreamSynchronize(b->stream));
-    const int64_t P = (int64_t)b->nx[g] * b->ny[g];
-    std::fill(rho, rho + P, 0.0);
-    std::fill(ux, ux + P, 0.0);
-    std::fill(uy, uy + P, 0.0);
     const auto& cp = b->cellPos[g];
-    for (int64_t c = 0; c < n; c++) {
-        rho[cp[c]] = b->ph.rhoin + (double)h[c];
-        ux[cp[c]] = h[n + c];
-        uy[cp[c]] = h[2 * n + c];
+    const double rho0 = b->ph.rhoin;
+    const int64_t P = (int64_t)b->nx[g] * b->ny[g];
+    auto clear = [&](int64_t p0, int64_t p1) {
+        std::fill(rho + p0, rho + p1, 0.0);
+        std::fill(ux + p0, ux + p1, 0.0);
+        std::fill(uy + p0, uy + p1, 0.0);
+    };
+    // cells [c0, c1) from their three planes in `from`.  Row-major cells: the
+    // sites from the first to the next range's first are theirs to clear;
+    // tile-major ones are cleared beforehand.
+    if (b->tiled || n == 0) clear(0, P);
+    auto put = [&](int64_t c0, int64_t c1, const float* from) {
+        if (!b->tiled) clear(c0 ? cp[c0] : 0, c1 < n ? cp[c1] : P);
+        const float *r = from - c0, *x = r + (c1 - c0), *y = x + (c1 - c0);
+        for (int64_t c = c0; c < c1; c++) {
+            rho[cp[c]] = rho0 + (double)r[c];
+            ux[cp[c]] = x[c];
+            uy[cp[c]] = y[c];
+        }
+    };
+    auto fetch = [&](float* to, int64_t c0, int64_t c1) -> hipError_t {
+        for (int k = 0; k < 3; k++) {
+            const hipError_t e = hipMemcpyAsync(to + k * (c1 - c0), b->mac + k * S + o + c0, (c1 - c0) * 4,
+                                                hipMemcpyDeviceToHost, b->stream);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    };
+    if ((size_t)n * 12 >= Readback::SLOT && b->readback.ready()) {
+        const int64_t per = (int64_t)(Readback::SLOT / 4 / 12) / 64 * 64;  // a quarter slot: work for every thread
+        BT_TRY(b->readback.each(b->prm.device, b->stream, (size_t)((n + per - 1) / per),
+                                [&](size_t i, char* slot) { return fetch((float*)slot, i * per, std::min<int64_t>(n, (i + 1) * per)); },
+                                [&](size_t i, const char* slot) { put(i * per, std::min<int64_t>(n, (i + 1) * per), (const float*)slot); }));
+        return MTS_OK;
     }
+    std::vector<float> h;
+    try {
+        h.resize(3 * n);
+    } catch (...) {
+        return set_error(MTS_ERR_OOM, "host allocation");
+    }
+    BT_TRY(fetch(h.data(), 0, n));
+    BT_TRY(hipStreamSynchronize(b->stream));
+    if (n) put(0, n, h.data());
     return MTS_OK;
 }
 

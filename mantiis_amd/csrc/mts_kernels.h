@@ -259,7 +259,12 @@ void launch_coarse_interp(hipStream_t st, int64_t nrows, const CoarseRow* rows, 
                           const double* usq2);
 void launch_fine_interp(hipStream_t st, int64_t nrows, const FineRow* rows, double* f1, int64_t stride1, const double* f2,
                         int64_t stride2, const double* rho1, const double* ux1, const double* uy1, const double* usq1);
-void launch_pixel_out(hipStream_t st, int64_t npix, const int64_t* src, const double* const* level_arrays, double* out);
+// Level fields and the three pixel images (ux, uy, rho) formed from them.
+struct PixelSpec {
+    const double *ux[MTS_MAX_LEVELS] = {}, *uy[MTS_MAX_LEVELS] = {}, *rho[MTS_MAX_LEVELS] = {};
+    double* out[3] = {};
+};
+void launch_pixel_out(hipStream_t st, int64_t npix, const uint8_t* level, const int32_t* site, const PixelSpec& s);
 // Unfused LB2D methods on the canonical FP64 arrays (mts_phase.hip).
 struct PhaseArrays {
     double *f, *ftemp, *feq, *fneq, *fb;

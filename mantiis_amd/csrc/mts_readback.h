@@ -1,0 +1,141 @@
+// Field readback: device arrays to the caller's (pageable) arrays.
+//
+// A plain copy to pageable memory is staged by the runtime on one thread,
+// copy and page faults one after the other: 10.6 GB/s measured for the three
+// fields of a 3000 x 2600 lattice (187 MB, 17.7 ms of a 112 ms call).  Here a
+// few host threads each own one pinned slot, take the next chunk, bring it
+// over on the handle's stream and move it to its destination while the other
+// threads' chunks cross the bus.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <functional>
+#include <thread>
+#include <vector>
+
+namespace mts {
+
+// Runs work(0) .. work(n - 1) on up to n host threads, the caller's among
+// them.  A thread that cannot be started leaves its share to the others: work
+// items are taken from a common counter by whoever runs.
+inline void on_threads(int n, const std::function<void(int)>& work) {
+    std::vector<std::thread> pool;
+    for (int t = 1; t < n; t++) {
+        try {
+            pool.emplace_back(work, t);
+        } catch (...) {
+            break;
+        }
+    }
+    work(0);
+    for (auto& t : pool) t.join();
+}
+inline int host_threads() { return std::max(1, std::min(8, (int)std::thread::hardware_concurrency())); }
+
+class Readback {
+  public:
+    struct Piece {
+        void* dst;
+        const void* src;
+        size_t bytes;
+    };
+    static constexpr size_t SLOT = (size_t)1 << 20;  // bytes per thread: 8 MB pinned per handle
+    static constexpr size_t MIN_BYTES = (size_t)2 << 20;  // below, a plain copy is as fast
+
+    // Pins the slots (a handle whose fields are large does so when it is made).
+    bool ready() {
+        if (pin_) return true;
+        if (failed_) return false;
+        slots_ = host_threads();
+        if (hipHostMalloc((void**)&pin_, slots_ * SLOT, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            pin_ = nullptr;
+            failed_ = true;
+            return false;
+        }
+        ev_.assign(slots_, nullptr);
+        for (hipEvent_t& e : ev_)
+            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                e = nullptr;
+                release();
+                failed_ = true;
+                return false;
+            }
+        return true;
+    }
+    // Copies the pieces (device to host) behind the work of `stream` and
+    // returns when they are there.
+    hipError_t run(int device, hipStream_t stream, const std::vector<Piece>& pieces) {
+        size_t total = 0;
+        std::vector<size_t> first(1, 0);  // chunks before piece i
+        for (const Piece& p : pieces) {
+            total += p.bytes;
+            first.push_back(first.back() + (p.bytes + SLOT - 1) / SLOT);
+        }
+        if (total < MIN_BYTES || !ready()) {
+            for (const Piece& p : pieces) {
+                const hipError_t e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+                if (e != hipSuccess) return e;
+            }
+            return hipStreamSynchronize(stream);
+        }
+        auto at = [&](size_t c, size_t& i, size_t& off) -> size_t {
+            i = std::upper_bound(first.begin(), first.end(), c) - first.begin() - 1;
+            off = (c - first[i]) * SLOT;
+            return std::min(SLOT, pieces[i].bytes - off);
+        };
+        return each(
+            device, stream, first.back(),
+            [&](size_t c, char* slot) {
+                size_t i, off;
+                const size_t n = at(c, i, off);
+                return hipMemcpyAsync(slot, (const char*)pieces[i].src + off, n, hipMemcpyDeviceToHost, stream);
+            },
+            [&](size_t c, const char* slot) {
+                size_t i, off;
+                const size_t n = at(c, i, off);
+                std::memcpy((char*)pieces[i].dst + off, slot, n);
+            });
+    }
+    // n chunks on the slots' threads (ready() must hold): fetch(i, slot) queues
+    // the copies of chunk i into the slot on `stream`, take(i, slot) uses it
+    // when they are done.
+    template <class Fetch, class Take>
+    hipError_t each(int device, hipStream_t stream, size_t n, Fetch fetch, Take take) {
+        std::atomic<size_t> next{0};
+        std::atomic<int> err{(int)hipSuccess};
+        on_threads((int)std::min<size_t>(slots_, n), [&](int t) {
+            hipError_t e = hipSetDevice(device);
+            char* slot = pin_ + (size_t)t * SLOT;
+            for (size_t c; e == hipSuccess && (c = next.fetch_add(1)) < n;) {
+                e = fetch(c, slot);
+                if (e == hipSuccess) e = hipEventRecord(ev_[t], stream);
+                if (e == hipSuccess) e = hipEventSynchronize(ev_[t]);
+                if (e == hipSuccess) take(c, slot);
+            }
+            if (e != hipSuccess) err = (int)e;
+        });
+        if (err.load() != (int)hipSuccess) (void)hipStreamSynchronize(stream);  // no copy into a slot is left behind
+        return (hipError_t)err.load();
+    }
+    void release() {
+        for (hipEvent_t e : ev_)
+            if (e) (void)hipEventDestroy(e);
+        ev_.clear();
+        if (pin_) (void)hipHostFree(pin_);
+        pin_ = nullptr;
+    }
+    ~Readback() { release(); }
+
+  private:
+    char* pin_ = nullptr;
+    std::vector<hipEvent_t> ev_;
+    int slots_ = 0;
+    bool failed_ = false;
+};
+
+}  // namespace mts

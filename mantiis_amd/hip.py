@@ -242,7 +242,7 @@ class Lattice:
 
     def complete_domain(self):
         n = self.nx * self.ny
-        ux, uy, rho = np.zeros(n), np.zeros(n), np.zeros(n)
+        ux, uy, rho = np.empty(n), np.empty(n), np.empty(n)  # written whole
         _check(self.lib, self.lib.mts_complete_domain(self.h, _p(ux, _D), _p(uy, _D), _p(rho, _D)))
         return ux, uy, rho
 
@@ -429,7 +429,7 @@ class Batch:
 
     def fields(self, g):
         shp = self.shapes[g]
-        rho, ux, uy = (np.zeros(shp) for _ in range(3))
+        rho, ux, uy = (np.empty(shp) for _ in range(3))  # written whole
         _check(self.lib, self.lib.mts_batch_fields(self.h, int(g), _p(rho, _D), _p(ux, _D), _p(uy, _D)))
         return rho, ux, uy
 
