@@ -243,11 +243,13 @@ inline size_t conv_lds(int Cin, int ksz, int steps, int rows) {
 // one step whose eight elements per lane are picked one by one.
 //
 // Bound: the LDS reads of the pixel operand (one 16-byte read per lane feeds
-// NTW products) and, in the deep layers, the weights' way through the L1;
-// weights are read ahead by two steps.  The 64x64 implicit GEMM it replaces
-// fetched every input element nine times through per-element index divisions:
-// predicting four 512 x 512 images took 1.70 ms, a training step on eight
-// 256 x 256 images 5.0 ms.
+// NTW products) and the weights' way through the L1 (one read feeds MTW); with
+// offsets, weights and pixels read when they were used, every step waited for
+// the LDS twice: predicting four 512 x 512 images (191 GFLOP) took 767 us
+// against 610 with them read ahead.  The 64x64 implicit GEMM before it, which
+// fetched every input element nine times through per-element index divisions,
+// took 1703 us; a training step on eight 256 x 256 images went from 5.02 to
+// 2.08 ms with k_convw.
 template <int MTW, int NTW, int WM, int WN>
 __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
     extern __shared__ char lds[];
@@ -304,32 +306,55 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
         for (int n = 0; n < NTW; n++) acc[m][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // weights of step k: CH tiles of 64 lanes x 8 elements
     const bf16x8* wp = (const bf16x8*)a.Wf + ((int64_t)blockIdx.y * a.steps * CH + wn * NTW) * 64 + l;
-    bf16x8 wr[3][NTW];
-#pragma unroll
-    for (int u = 0; u < 2; u++)
-        if (u < a.steps)
-#pragma unroll
-            for (int n = 0; n < NTW; n++) wr[u][n] = wp[(u * CH + n) * 64];
-    __syncthreads();
     const char* px0 = tile + ((wm * MTW) * LW + i) * PS;
-    for (int k0 = 0; k0 < a.steps; k0 += 3) {
+    if (!a.direct && !small) {
+        // Weights and offsets are read two steps ahead and pixels one, so that
+        // a step's products wait for nothing they have just asked for; the
+        // rings' places are fixed by unrolling six steps.
+        bf16x8 wr[3][NTW], xf[2][MTW];
+        int of[3];
 #pragma unroll
-        for (int u = 0; u < 3; u++) {
-            const int k = k0 + u;
-            if (k >= a.steps) break;
-            if (k + 2 < a.steps)
+        for (int u = 0; u < 2; u++)
+            if (u < a.steps)
 #pragma unroll
-                for (int n = 0; n < NTW; n++) wr[(u + 2) % 3][n] = wp[((k + 2) * CH + n) * 64];
+                for (int n = 0; n < NTW; n++) wr[u][n] = wp[(u * CH + n) * 64];
+        __syncthreads();
+        of[0] = s_off[q];
+        of[1] = s_off[a.steps > 1 ? 4 + q : q];
+#pragma unroll
+        for (int m = 0; m < MTW; m++) xf[0][m] = *(const bf16x8*)(px0 + m * LW * PS + of[0]);
+        for (int k0 = 0; k0 < a.steps; k0 += 6) {
+#pragma unroll
+            for (int u = 0; u < 6; u++) {
+                const int k = k0 + u;
+                if (k >= a.steps) break;
+                if (k + 2 < a.steps) {
+#pragma unroll
+                    for (int n = 0; n < NTW; n++) wr[(u + 2) % 3][n] = wp[((k + 2) * CH + n) * 64];
+                    of[(u + 2) % 3] = s_off[4 * (k + 2) + q];
+                }
+                if (k + 1 < a.steps) {
+                    const int o = of[(u + 1) % 3];
+#pragma unroll
+                    for (int m = 0; m < MTW; m++) xf[(u + 1) % 2][m] = *(const bf16x8*)(px0 + m * LW * PS + o);
+                }
+                // lanes past the last group hold zeros (their weights are zero,
+                // but an infinite activation would make a NaN of the product)
+                if (4 * k + 3 >= ng && 4 * k + q >= ng)
+#pragma unroll
+                    for (int m = 0; m < MTW; m++) xf[u % 2][m] = bf16x8{};
+#pragma unroll
+                for (int n = 0; n < NTW; n++)
+#pragma unroll
+                    for (int m = 0; m < MTW; m++)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u % 3][n], xf[u % 2][m], acc[m][n], 0, 0, 0);
+            }
+        }
+    } else {
+        __syncthreads();
+        for (int k = 0; k < a.steps; k++) {
             bf16x8 xf[MTW];
-            if (a.direct) {
-                const int g = 4 * k + q, kk = min(g / C8, a.ksz * a.ksz - 1), c8 = g - g / C8 * C8;
-                int dy, dx;
-                koff(kk, a.ksz, dy, dx);
-#pragma unroll
-                for (int m = 0; m < MTW; m++)
-                    xf[m] = *(const bf16x8*)a.in.at(b, wrapn(y0 + wm * MTW + m + a.sgn * dy, H),
-                                                    wrapn(x0 + i + a.sgn * dx, W), c8 * 8);
-            } else if (small) {
+            if (small) {
 #pragma unroll
                 for (int m = 0; m < MTW; m++)
 #pragma unroll
@@ -338,20 +363,23 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
                         xf[m][e] = 8 * q + e < ng ? v : (bf16)0.0f;
                     }
             } else {
-                const int o = s_off[4 * k + q];
+                const int g = 4 * k + q, kk = min(g / C8, a.ksz * a.ksz - 1), c8 = g - g / C8 * C8;
+                int dy, dx;
+                koff(kk, a.ksz, dy, dx);
 #pragma unroll
-                for (int m = 0; m < MTW; m++) xf[m] = *(const bf16x8*)(px0 + m * LW * PS + o);
+                for (int m = 0; m < MTW; m++) {
+                    const bf16x8 v = *(const bf16x8*)a.in.at(b, wrapn(y0 + wm * MTW + m + a.sgn * dy, H),
+                                                             wrapn(x0 + i + a.sgn * dx, W), c8 * 8);
+                    xf[m] = g < ng ? v : bf16x8{};
+                }
             }
-            // lanes past the last group hold zeros (their weights are zero, but
-            // an infinite activation would make a NaN of the product)
-            if (!small && 4 * k + 3 >= ng && 4 * k + q >= ng)
 #pragma unroll
-                for (int m = 0; m < MTW; m++) xf[m] = bf16x8{};
-#pragma unroll
-            for (int n = 0; n < NTW; n++)
+            for (int n = 0; n < NTW; n++) {
+                const bf16x8 wv = wp[(k * CH + n) * 64];
 #pragma unroll
                 for (int m = 0; m < MTW; m++)
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u][n], xf[m], acc[m][n], 0, 0, 0);
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, xf[m], acc[m][n], 0, 0, 0);
+            }
         }
     }
     // lane (i, q) holds channels 4 q .. + 3 of pixel i of each row
