@@ -813,23 +813,27 @@ static int create_multi(mts_sim_s* s, int nx, int ny, const int32_t* pore, const
         const size_t np = (size_t)nx * ny;
         std::vector<uint8_t> lev(np, 0);
         std::vector<int32_t> site(np, 0);
-        for (int64_t c = 0; c < s->mg.ncell; c++) {
-            if (s->mg.isBuffer[c]) continue;
-            const int l = s->mg.level[c] - 1, w = 1 << l;
-            const int32_t q = (int32_t)((int64_t)(s->mg.cy[c] >> l) * s->lv[l].nx + (s->mg.cx[c] >> l));
-            for (int dy = 0; dy < w; dy++)
-                for (int dx = 0; dx < w; dx++) {
-                    const size_t p = (size_t)(s->mg.cy[c] + dy) * nx + s->mg.cx[c] + dx;
-                    lev[p] = (uint8_t)(l + 1);
-                    site[p] = q;
+        const int nt = np < 65536 ? 1 : host_threads();
+        std::atomic<int> next{0};
+        on_threads(nt, [&](int) {  // non-buffer cells cover disjoint pixels
+            for (int k; (k = next.fetch_add(1)) < nt;)
+                for (int64_t c = s->mg.ncell * k / nt; c < s->mg.ncell * (k + 1) / nt; c++) {
+                    if (s->mg.isBuffer[c]) continue;
+                    const int l = s->mg.level[c] - 1, w = 1 << l;
+                    const int32_t q = (int32_t)((int64_t)(s->mg.cy[c] >> l) * s->lv[l].nx + (s->mg.cx[c] >> l));
+                    for (int dy = 0; dy < w; dy++)
+                        for (int dx = 0; dx < w; dx++) {
+                            const size_t p = (size_t)(s->mg.cy[c] + dy) * nx + s->mg.cx[c] + dx;
+                            lev[p] = (uint8_t)(l + 1);
+                            site[p] = q;
+                        }
                 }
-        }
+        });
         if ((rc = s->alloc(&s->d_pixLevel, np)) || (rc = s->alloc(&s->d_pixSite, np)) ||
             (rc = upload(s->d_pixLevel, lev.data(), np, s->stream)) ||
             (rc = upload(s->d_pixSite, site.data(), np * 4, s->stream)))
             return rc;
         HIP_TRY(hipStreamSynchronize(s->stream));  // the host maps go out of scope
-        if (np * 24 >= Readback::MIN_BYTES) (void)s->readback.ready();
     }
     upload_icsr(s->stream);
     upload_xynorm(s->stream);
@@ -1244,7 +1248,6 @@ int mts_create(int nx, int ny, const int32_t* pore, const double* kn, const doub
     upload_icsr(s->stream);
     upload_xynorm(s->stream);
     *out = s;
-    if ((size_t)s->P * 24 >= Readback::MIN_BYTES) (void)s->readback.ready();
     rc = mts_initialize(s);
     if (rc) {
         *out = nullptr;

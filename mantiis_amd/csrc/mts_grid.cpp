@@ -337,8 +337,8 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
         // population opp(j) reaches no other cell: its plane holds the fed
         // value between passes.  Its specular sources are those of its type
         // (the kernels' table).  Cells that break this are RAW.
-        bool irregular = wall != 0 && spec != ci.spec[t];
-        for (int j = 1; j < 9; j++) {
+        bool irregular = wall != 0 ? spec != ci.spec[t] : in != 0xffu;
+        for (int j = 1; wall != 0 && j < 9; j++) {
             const bool inj = (in >> (j - 1)) & 1u, fed = (wall >> (OPP[j] - 1)) & 1u;
             if (inj == fed || (inj && ((spec >> (4 * (j - 1))) & 15u))) irregular = true;
             if (!((wall >> (j - 1)) & 1u)) continue;

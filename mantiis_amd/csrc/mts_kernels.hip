@@ -98,10 +98,11 @@ struct Lat {
     }
 };
 
-// Populations are read by the neighbours' threads too: loads are cached, stores
-// stream past the caches (the next read is a full step later).
+// Populations stay in the caches: the small FP64 lattices fit there until the
+// next step (100 x 100 Shan-Chen 1.00 -> 0.95 ms per 100 steps against
+// nontemporal stores, 64 x 64 transport 589 -> 575 us).
 __device__ __forceinline__ double ld64(const double* __restrict__ a, int64_t i) { return a[i]; }
-__device__ __forceinline__ void st64(double* __restrict__ a, int64_t i, double v) { __builtin_nontemporal_store(v, a + i); }
+__device__ __forceinline__ void st64(double* __restrict__ a, int64_t i, double v) { a[i] = v; }
 
 // ============================================================================
 // FP64 reference-order arithmetic.  The reference evaluates dense 9x9

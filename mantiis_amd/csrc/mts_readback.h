@@ -42,10 +42,10 @@ class Readback {
         const void* src;
         size_t bytes;
     };
-    static constexpr size_t SLOT = (size_t)1 << 20;  // bytes per thread: 8 MB pinned per handle
+    static constexpr size_t SLOT = (size_t)1 << 20;  // bytes per thread: 8 MB pinned per handle (256 KB slots read at half the rate)
     static constexpr size_t MIN_BYTES = (size_t)2 << 20;  // below, a plain copy is as fast
 
-    // Pins the slots (a handle whose fields are large does so when it is made).
+    // Pins the slots, at the first read that is large enough.
     bool ready() {
         if (pin_) return true;
         if (failed_) return false;
