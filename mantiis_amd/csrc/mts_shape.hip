@@ -51,9 +51,14 @@ typedef unsigned long long u64;
 constexpr int THIN_S = 32;                     // subiterations per launch (even)
 constexpr int THIN_TW = 2;                     // inner tile width, words
 constexpr int THIN_TH = 64;                    // inner tile height, rows
-constexpr int THIN_LW = THIN_TW + 2;           // LDS words per row (one halo word each side)
+// A thread holds 32 pixels: the halo left and right is one half word (it only
+// has to cover THIN_S pixels), and the deletion rule, a serial chain of bitwise
+// steps, runs once per subiteration; with 64-bit words it ran twice, on a halo
+// twice as wide.
+constexpr int THIN_LW = 2 * THIN_TW + 2;       // half words per row (one of halo each side)
 constexpr int THIN_LR = THIN_TH + 2 * THIN_S;  // LDS rows
-constexpr int THIN_THREADS = THIN_LW * THIN_LR;  // one word per thread
+constexpr int THIN_THREADS = THIN_LW * THIN_LR;  // one half word per thread
+static_assert(THIN_S <= 32, "one half word of halo");
 static_assert(THIN_S % 2 == 0 && THIN_THREADS <= 1024, "tile shape");
 static_assert(THIN_S < THIN_TH && THIN_S < 64 * THIN_TW, "a launch's reach must stay inside the neighbour tiles");
 constexpr int SEG = 32;                      // rows per column chunk
@@ -160,27 +165,16 @@ __device__ __forceinline__ uint32_t zs_keep(uint32_t p0, uint32_t p1, uint32_t p
     return op3<L_ANDN>(me, del, 0u);
 }
 
-template <int SUB>
-__device__ __forceinline__ u64 zs_keep64(u64 p0, u64 p1, u64 p2, u64 p3, u64 p4, u64 p5, u64 p6, u64 p7, u64 me,
-                                         u64 mask) {
-    const uint32_t lo = zs_keep<SUB>((uint32_t)p0, (uint32_t)p1, (uint32_t)p2, (uint32_t)p3, (uint32_t)p4,
-                                     (uint32_t)p5, (uint32_t)p6, (uint32_t)p7, (uint32_t)me, (uint32_t)mask);
-    const uint32_t hi = zs_keep<SUB>((uint32_t)(p0 >> 32), (uint32_t)(p1 >> 32), (uint32_t)(p2 >> 32),
-                                     (uint32_t)(p3 >> 32), (uint32_t)(p4 >> 32), (uint32_t)(p5 >> 32),
-                                     (uint32_t)(p6 >> 32), (uint32_t)(p7 >> 32), (uint32_t)(me >> 32),
-                                     (uint32_t)(mask >> 32));
-    return (u64)hi << 32 | lo;
-}
-
 // THIN_S Zhang-Suen subiterations (starting with subiteration 0) of one
 // tile; out receives the inner tile.  Thinning only deletes, and one launch
 // moves information at most THIN_S pixels, so a tile whose 3 x 3 tile
 // neighbourhood did not change in the previous launch cannot change in this
 // one: it is skipped, and both ping-pong buffers already hold it (it was
 // unchanged, or skipped, the launch before).  chgIn / chgOut: per tile,
-// changed in the previous / this launch; cnt counts changed tiles.
+// changed in the previous / this launch; cnt (optional) counts changed tiles.
+// in / out: the canvas words as NH half words per row (bits 0..31 first).
 __global__ void __launch_bounds__(THIN_THREADS)
-    k_thin(const u64* __restrict__ in, u64* __restrict__ out, int H, int Wc, int WW, int tilesX, int tilesY,
+    k_thin(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int H, int Wc, int NH, int tilesX, int tilesY,
            const uint8_t* __restrict__ chgIn, uint8_t* __restrict__ chgOut, unsigned* __restrict__ cnt) {
     const int bx = blockIdx.x, by = blockIdx.y;
     bool live = false;
@@ -199,64 +193,64 @@ __global__ void __launch_bounds__(THIN_THREADS)
     // halo; it holds set pixels, so that a fluid halo next to it is a full
     // neighbourhood the early-out below skips rather than a false edge that
     // erodes on every subiteration.
-    __shared__ u64 L[2][THIN_LR + 2][THIN_LW + 2];
+    __shared__ uint32_t L[2][THIN_LR + 2][THIN_LW + 2];
     const int t = threadIdx.x;
     for (int e = t; e < 2 * (THIN_LR + 2); e += THIN_THREADS) {
-        L[e & 1][e >> 1][0] = ~0ull;
-        L[e & 1][e >> 1][THIN_LW + 1] = ~0ull;
+        L[e & 1][e >> 1][0] = ~0u;
+        L[e & 1][e >> 1][THIN_LW + 1] = ~0u;
     }
     for (int e = t; e < 2 * THIN_LW; e += THIN_THREADS) {
         const int b = e / THIN_LW, c = e % THIN_LW + 1;
-        L[b][0][c] = ~0ull;
-        L[b][THIN_LR + 1][c] = ~0ull;
+        L[b][0][c] = ~0u;
+        L[b][THIN_LR + 1][c] = ~0u;
     }
     const int lc = t % THIN_LW, lr = t / THIN_LW;
-    const int gw = bx * THIN_TW - 1 + lc;
+    const int gw = bx * 2 * THIN_TW - 1 + lc;
     const int gr = by * THIN_TH - THIN_S + lr;
-    const bool inimg = gr >= 0 && gr < H && gw >= 0 && gw < WW;
-    const u64 orig = inimg ? in[(size_t)gr * WW + gw] : 0ull;
+    const bool inimg = gr >= 0 && gr < H && gw >= 0 && gw < NH;
+    const uint32_t orig = inimg ? in[(size_t)gr * NH + gw] : 0u;
     // pixels that may be deleted: image rows 1..H-2, columns 1..Wc-2
-    u64 mask = 0;
+    uint32_t mask = 0;
     if (inimg && gr >= 1 && gr <= H - 2) {
-        const int lo = max(1 - 64 * gw, 0), hi = min(Wc - 2 - 64 * gw, 63);
-        if (lo <= hi) mask = (hi == 63 ? ~0ull : ((1ull << (hi + 1)) - 1)) & ~((1ull << lo) - 1);
+        const int lo = max(1 - 32 * gw, 0), hi = min(Wc - 2 - 32 * gw, 31);
+        if (lo <= hi) mask = (hi == 31 ? ~0u : ((1u << (hi + 1)) - 1)) & ~((1u << lo) - 1);
     }
-    u64 me = orig;
+    uint32_t me = orig;
     L[0][lr + 1][lc + 1] = me;
     __syncthreads();
 #pragma unroll 2
     for (int sub = 0; sub < THIN_S; sub++) {
         const int cur = sub & 1;
-        const u64 up = L[cur][lr][lc + 1], dn = L[cur][lr + 2][lc + 1];
-        const u64 upL = L[cur][lr][lc], upR = L[cur][lr][lc + 2];
-        const u64 meL = L[cur][lr + 1][lc], meR = L[cur][lr + 1][lc + 2];
-        const u64 dnL = L[cur][lr + 2][lc], dnR = L[cur][lr + 2][lc + 2];
+        const uint32_t up = L[cur][lr][lc + 1], dn = L[cur][lr + 2][lc + 1];
+        const uint32_t upL = L[cur][lr][lc], upR = L[cur][lr][lc + 2];
+        const uint32_t meL = L[cur][lr + 1][lc], meR = L[cur][lr + 1][lc + 2];
+        const uint32_t dnL = L[cur][lr + 2][lc], dnR = L[cur][lr + 2][lc + 2];
         // nothing to delete in a word without deletable set pixels, or whose
         // whole neighbourhood is set (B = 8): whole waves skip the rule
-        if ((me & mask) != 0 && (me & up & dn & upL & upR & meL & meR & dnL & dnR) != ~0ull) {
+        if ((me & mask) != 0 && (me & up & dn & upL & upR & meL & meR & dnL & dnR) != ~0u) {
             // neighbour ring N, NE, E, SE, S, SW, W, NW (value of the pixel
             // one column right: word >> 1 with the next word's bit 0 on top)
-            const u64 p0 = up;
-            const u64 p1 = (up >> 1) | (upR << 63);
-            const u64 p2 = (me >> 1) | (meR << 63);
-            const u64 p3 = (dn >> 1) | (dnR << 63);
-            const u64 p4 = dn;
-            const u64 p5 = (dn << 1) | (dnL >> 63);
-            const u64 p6 = (me << 1) | (meL >> 63);
-            const u64 p7 = (up << 1) | (upL >> 63);
-            me = cur == 0 ? zs_keep64<0>(p0, p1, p2, p3, p4, p5, p6, p7, me, mask)
-                          : zs_keep64<1>(p0, p1, p2, p3, p4, p5, p6, p7, me, mask);
+            const uint32_t p0 = up;
+            const uint32_t p1 = (up >> 1) | (upR << 31);
+            const uint32_t p2 = (me >> 1) | (meR << 31);
+            const uint32_t p3 = (dn >> 1) | (dnR << 31);
+            const uint32_t p4 = dn;
+            const uint32_t p5 = (dn << 1) | (dnL >> 31);
+            const uint32_t p6 = (me << 1) | (meL >> 31);
+            const uint32_t p7 = (up << 1) | (upL >> 31);
+            me = cur == 0 ? zs_keep<0>(p0, p1, p2, p3, p4, p5, p6, p7, me, mask)
+                          : zs_keep<1>(p0, p1, p2, p3, p4, p5, p6, p7, me, mask);
         }
         L[cur ^ 1][lr + 1][lc + 1] = me;
         __syncthreads();
     }
-    const bool inner = inimg && lr >= THIN_S && lr < THIN_S + THIN_TH && lc >= 1 && lc <= THIN_TW;
-    if (inner) out[(size_t)gr * WW + gw] = me;
+    const bool inner = inimg && lr >= THIN_S && lr < THIN_S + THIN_TH && lc >= 1 && lc <= 2 * THIN_TW;
+    if (inner) out[(size_t)gr * NH + gw] = me;
     const bool changed = inner && me != orig;
     const bool any = __syncthreads_or(changed);
     if (t == 0) {
         chgOut[by * tilesX + bx] = any ? 1 : 0;
-        if (any) atomicAdd(cnt, 1u);
+        if (any && cnt) atomicAdd(cnt, 1u);
     }
 }
 
@@ -273,88 +267,97 @@ __global__ void k_crop(const u64* __restrict__ cv, int WW, int m, int nx, int ny
 // z = 1: skeleton, zero where the byte is set).
 __device__ __forceinline__ bool zero_at(const uint8_t* img, int z, size_t p) { return z ? img[p] != 0 : img[p] == 0; }
 
+// Zero pixels of column j in the SEG rows from r0 on, bit k for row r0 + k:
+// the rows' loads are independent, and neighbouring threads read neighbouring
+// columns.
+static_assert(SEG == 32, "a chunk's zeros are one word");
+__device__ __forceinline__ uint32_t chunk_zeros(const uint8_t* img, int z, int nx, int ny, int j, int r0) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < SEG; k++)
+        if (r0 + k < ny && zero_at(img, z, (size_t)(r0 + k) * nx + j)) m |= 1u << k;
+    return m;
+}
+
 // Per column chunk of SEG rows: its first and last zero row (-1: none).
 __global__ void k_colseg(const uint8_t* __restrict__ dom, const uint8_t* __restrict__ skel, int nx, int ny,
                          int nseg, int* __restrict__ first, int* __restrict__ last) {
     const int z = blockIdx.y;
-    const uint8_t* img = z ? skel : dom;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (int64_t)nseg * nx) return;
-    const int sg = (int)(t / nx), j = (int)(t % nx);
-    const int r0 = sg * SEG, r1 = min(r0 + SEG, ny);
-    int f = -1, l = -1;
-    for (int r = r0; r < r1; r++)
-        if (zero_at(img, z, (size_t)r * nx + j)) {
-            if (f < 0) f = r;
-            l = r;
-        }
+    const int sg = (int)(t / nx), j = (int)(t % nx), r0 = sg * SEG;
+    const uint32_t m = chunk_zeros(z ? skel : dom, z, nx, ny, j, r0);
     const size_t o = (size_t)z * nseg * nx + t;
-    first[o] = f;
-    last[o] = l;
+    first[o] = m ? r0 + __ffs((int)m) - 1 : -1;
+    last[o] = m ? r0 + 31 - __clz((int)m) : -1;
 }
 
-// Distance in its column from every pixel to the nearest zero (-1: none),
-// and that zero's row (the upper one of two at the same distance).
+// Row of the nearest zero of its column for every pixel (-1: none; the upper
+// one of two at the same distance).  A thread takes a chunk's SEG pixels: the
+// chunk's zeros as one word, the nearest ones outside from the chunk summaries.
+// One thread per pixel, scanning up and down, took 40 us for 1024 x 1024.
 __global__ void k_colpass(const uint8_t* __restrict__ dom, const uint8_t* __restrict__ skel, int nx, int ny,
                           int nseg, const int* __restrict__ first, const int* __restrict__ last,
-                          int* __restrict__ g, int* __restrict__ zrow) {
+                          int* __restrict__ zrow) {
     const int z = blockIdx.y;
-    const uint8_t* img = z ? skel : dom;
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (int64_t)nx * ny) return;
-    const int i = (int)(p / nx), j = (int)(p % nx);
-    const int sg = i / SEG;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)nseg * nx) return;
+    const int sg = (int)(t / nx), j = (int)(t % nx), r0 = sg * SEG;
+    const uint32_t m = chunk_zeros(z ? skel : dom, z, nx, ny, j, r0);
     const int* F = first + (size_t)z * nseg * nx;
     const int* Ls = last + (size_t)z * nseg * nx;
-    int up = -1, dn = -1;
-    for (int r = i; r >= sg * SEG; r--)
-        if (zero_at(img, z, (size_t)r * nx + j)) {
-            up = r;
-            break;
-        }
-    for (int s = sg - 1; up < 0 && s >= 0; s--) up = Ls[(size_t)s * nx + j];
-    const int r1 = min((sg + 1) * SEG, ny);
-    for (int r = i; r < r1; r++)
-        if (zero_at(img, z, (size_t)r * nx + j)) {
-            dn = r;
-            break;
-        }
-    for (int s = sg + 1; dn < 0 && s < nseg; s++) dn = F[(size_t)s * nx + j];
-    const int zr = up >= 0 && (dn < 0 || i - up <= dn - i) ? up : dn;
-    g[(size_t)z * nx * ny + p] = zr < 0 ? -1 : (zr <= i ? i - zr : zr - i);
-    zrow[(size_t)z * nx * ny + p] = zr;
+    int above = -1, below = -1;
+    for (int s = sg - 1; above < 0 && s >= 0; s--) above = Ls[(size_t)s * nx + j];
+    for (int s = sg + 1; below < 0 && s < nseg; s++) below = F[(size_t)s * nx + j];
+    int* out = zrow + (size_t)z * nx * ny + j;
+#pragma unroll
+    for (int k = 0; k < SEG; k++) {
+        const int i = r0 + k;
+        if (i >= ny) break;
+        const uint32_t lo = m & (k == 31 ? ~0u : (2u << k) - 1), hi = m >> k;
+        const int up = lo ? r0 + 31 - __clz((int)lo) : above;
+        const int dn = hi ? i + __ffs((int)hi) - 1 : below;
+        out[(size_t)i * nx] = up >= 0 && (dn < 0 || i - up <= dn - i) ? up : dn;
+    }
 }
 
-// Squared distance to the nearest zero: min over the row of dx^2 + g^2
-// (-1: the image has no zero pixel), and for the skeleton image the index of
-// the first nearest zero in row-major order (ties resolved on (row, col):
-// within a column only the column's nearest zero can reach the minimum).
-__global__ void k_rowpass(const int* __restrict__ g, const int* __restrict__ zrow, int nx, int ny,
-                          int* __restrict__ k2, int* __restrict__ nearest) {
-    const int z = blockIdx.y;
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (int64_t)nx * ny) return;
-    const int i = (int)(p / nx), j = (int)(p % nx);
-    const int* row = g + (size_t)z * nx * ny + (size_t)i * nx;
-    const int* zr = zrow + (size_t)z * nx * ny + (size_t)i * nx;
-    const int64_t NONE = INT64_MAX;
-    int64_t best = NONE, bq = INT64_MAX;
-    auto consider = [&](int k, int64_t dx2) {
-        if (row[k] < 0) return;
-        const int64_t v = dx2 + (int64_t)row[k] * row[k], q = (int64_t)zr[k] * nx + k;
-        if (v < best || (v == best && q < bq)) {
+// Squared distance to the nearest zero: min over the row of dx^2 + g^2, g the
+// distance to the column's nearest zero (-1: the image has no zero pixel), and
+// for the skeleton image the index of the first nearest zero in row-major
+// order (ties resolved on (row, col): within a column only the column's nearest
+// zero can reach the minimum).  A block's pixels are in one row, whose columns'
+// zeros are in LDS; all values fit 32 bits (sides up to MAX_SIDE).  With the
+// row read from memory, distances and rows apart, it took 72 us for 1024^2.
+__global__ void __launch_bounds__(256) k_rowpass(const int* __restrict__ zrow, int nx, int ny, int* __restrict__ k2,
+                                                 int* __restrict__ nearest) {
+    static_assert(2 * (int64_t)MAX_SIDE * MAX_SIDE < INT32_MAX, "32-bit squared distances");
+    __shared__ int zr[MAX_SIDE];
+    const int z = blockIdx.z, i = blockIdx.y, j = blockIdx.x * 256 + threadIdx.x;
+    const int* row = zrow + ((size_t)z * ny + i) * nx;
+    for (int k = threadIdx.x; k < nx; k += 256) zr[k] = row[k];
+    __syncthreads();
+    if (j >= nx) return;
+    constexpr int NONE = INT32_MAX;
+    int best = NONE, bq = INT32_MAX;
+    auto consider = [&](int k, int dx2) {
+        const int r = zr[k];
+        if (r < 0) return;
+        const int v = dx2 + (i - r) * (i - r);
+        if (v > best) return;
+        const int q = r * nx + k;
+        if (v < best || q < bq) {
             best = v;
             bq = q;
         }
     };
     consider(j, 0);
-    for (int r = 1; r < nx && (int64_t)r * r <= best; r++) {
-        const int64_t r2 = (int64_t)r * r;
-        if (j - r >= 0) consider(j - r, r2);
-        if (j + r < nx) consider(j + r, r2);
+    for (int r = 1; r < nx && r * r <= best; r++) {
+        if (j - r >= 0) consider(j - r, r * r);
+        if (j + r < nx) consider(j + r, r * r);
     }
-    k2[(size_t)z * nx * ny + p] = best == NONE ? -1 : (int)best;
-    if (z == 1) nearest[p] = best == NONE ? -1 : (int)bq;
+    const size_t p = (size_t)i * nx + j;
+    k2[(size_t)z * nx * ny + p] = best == NONE ? -1 : best;
+    if (z == 1) nearest[p] = best == NONE ? -1 : bq;
 }
 
 // OpenCV's float value of a squared distance: sqrtf of the exact integer;
@@ -472,7 +475,7 @@ int grid_of(int64_t n, int b) { return (int)((n + b - 1) / b); }
 // mts_shape_create allocates them.
 struct ShapeLayout {
     int m, H, Wc, WW, nseg, tilesX, tilesY;
-    size_t cv0, cv1, skel, first, last, g, k2, zrow, nearest, cnt, chg, err, total;
+    size_t cv0, cv1, skel, first, last, k2, zrow, nearest, cnt, chg, err, total;
 };
 constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 constexpr ShapeLayout shape_layout(int nx, int ny) {
@@ -491,7 +494,6 @@ constexpr ShapeLayout shape_layout(int nx, int ny) {
     L.skel = o, o = align256(o + np);
     L.first = o, o = align256(o + 2 * (size_t)L.nseg * nx * sizeof(int));
     L.last = o, o = align256(o + 2 * (size_t)L.nseg * nx * sizeof(int));
-    L.g = o, o = align256(o + 2 * np * sizeof(int));
     L.k2 = o, o = align256(o + 2 * np * sizeof(int));
     L.zrow = o, o = align256(o + 2 * np * sizeof(int));
     L.nearest = o, o = align256(o + np * sizeof(int));
@@ -543,7 +545,6 @@ struct mts_shape_s {
     uint8_t* skel = nullptr;
     int* first = nullptr;
     int* last = nullptr;
-    int* g = nullptr;
     int* zrow = nullptr;
     int* k2 = nullptr;
     int* nearest = nullptr;
@@ -600,7 +601,6 @@ int mts_shape_create(int nx, int ny, mts_shape* out) {
     if (rc == MTS_OK) rc = h->alloc(&h->skel, np);
     if (rc == MTS_OK) rc = h->alloc(&h->first, 2 * (size_t)h->nseg * nx);
     if (rc == MTS_OK) rc = h->alloc(&h->last, 2 * (size_t)h->nseg * nx);
-    if (rc == MTS_OK) rc = h->alloc(&h->g, 2 * np);
     if (rc == MTS_OK) rc = h->alloc(&h->k2, 2 * np);
     if (rc == MTS_OK) rc = h->alloc(&h->zrow, 2 * np);
     if (rc == MTS_OK) rc = h->alloc(&h->nearest, np);
@@ -637,9 +637,6 @@ int mts_shape_run(mts_shape h, const uint8_t* domain, double resolution, double 
     k_canvas<<<grid_of(nw, 256), 256, 0, s>>>(domain, nx, ny, h->m, h->H, h->Wc, h->WW, h->cv[0], h->err);
     SH_TRY(hipGetLastError());
     int herr = 0;
-    SH_TRY(hipMemcpyAsync(&herr, h->err, sizeof(int), hipMemcpyDeviceToHost, s));
-    SH_TRY(hipStreamSynchronize(s));
-    if (herr & ERR_VALUE) return set_error(MTS_ERR_ARG, "mts_shape_run: domain values must be 0 or 1");
     // thinning: launches of THIN_S subiterations until one changes nothing;
     // every later launch would leave the image as it is
     const int ntiles = h->tilesX * h->tilesY;
@@ -647,23 +644,29 @@ int mts_shape_run(mts_shape h, const uint8_t* domain, double resolution, double 
     const int64_t maxLaunches = nw * 64 / (THIN_S / 2) + 2;  // each iteration but the last deletes a pixel
     k_fill8<<<grid_of(ntiles, 256), 256, 0, s>>>(h->chg, ntiles, 1);  // every tile is live in the first launch
     int cur = 0;
-    bool done = false;
+    bool done = false, checked = false;  // checked: the domain's values, with the first counters
     h->launches = 0;
     while (!done) {
         if (h->launches >= maxLaunches) return set_error(MTS_ERR_STATE, "mts_shape_run: thinning did not settle");
         k_fill8<<<1, 64, 0, s>>>((uint8_t*)h->cnt, CHECK_EVERY * sizeof(unsigned), 0);
-        for (int k = 0; k < CHECK_EVERY; k++) {
-            const int64_t l = h->launches + k;
-            k_thin<<<tg, THIN_THREADS, 0, s>>>(h->cv[cur], h->cv[cur ^ 1], h->H, h->Wc, h->WW, h->tilesX, h->tilesY,
-                                               h->chg + (l & 1) * ntiles, h->chg + ((l & 1) ^ 1) * ntiles,
-                                               h->cnt + k);
+        // The strip that continues the domain into the margins loses a row on
+        // each side per iteration for at least ny / 4 iterations, so nothing
+        // ends before launch ny / 64: no read until then.
+        const int64_t skip = h->launches == 0 ? std::max(ny / 64 / CHECK_EVERY - 1, 0) * CHECK_EVERY : 0;
+        for (int64_t k = -skip; k < CHECK_EVERY; k++) {
+            const int64_t l = h->launches++;
+            k_thin<<<tg, THIN_THREADS, 0, s>>>((const uint32_t*)h->cv[cur], (uint32_t*)h->cv[cur ^ 1], h->H, h->Wc,
+                                               2 * h->WW, h->tilesX, h->tilesY, h->chg + (l & 1) * ntiles,
+                                               h->chg + ((l & 1) ^ 1) * ntiles, k < 0 ? nullptr : h->cnt + k);
             cur ^= 1;
         }
         SH_TRY(hipGetLastError());
-        h->launches += CHECK_EVERY;
         unsigned c[CHECK_EVERY];
         SH_TRY(hipMemcpyAsync(c, h->cnt, sizeof(c), hipMemcpyDeviceToHost, s));
+        if (!checked) SH_TRY(hipMemcpyAsync(&herr, h->err, sizeof(int), hipMemcpyDeviceToHost, s));
         SH_TRY(hipStreamSynchronize(s));
+        checked = true;
+        if (herr & ERR_VALUE) return set_error(MTS_ERR_ARG, "mts_shape_run: domain values must be 0 or 1");
         for (int k = 0; k < CHECK_EVERY; k++) done |= c[k] == 0;
     }
     if (iterations) *iterations = (int)std::min<int64_t>(h->launches * (THIN_S / 2), INT32_MAX);
@@ -671,9 +674,9 @@ int mts_shape_run(mts_shape h, const uint8_t* domain, double resolution, double 
     k_crop<<<grid_of(np, 256), 256, 0, s>>>(h->cv[cur], h->WW, h->m, nx, ny, sk);
     k_colseg<<<dim3(grid_of((int64_t)h->nseg * nx, 256), 2), 256, 0, s>>>(domain, sk, nx, ny, h->nseg, h->first,
                                                                          h->last);
-    k_colpass<<<dim3(grid_of(np, 256), 2), 256, 0, s>>>(domain, sk, nx, ny, h->nseg, h->first, h->last, h->g,
-                                                        h->zrow);
-    k_rowpass<<<dim3(grid_of(np, 256), 2), 256, 0, s>>>(h->g, h->zrow, nx, ny, h->k2, h->nearest);
+    k_colpass<<<dim3(grid_of((int64_t)h->nseg * nx, 256), 2), 256, 0, s>>>(domain, sk, nx, ny, h->nseg, h->first,
+                                                                          h->last, h->zrow);
+    k_rowpass<<<dim3((nx + 255) / 256, ny, 2), 256, 0, s>>>(h->zrow, nx, ny, h->k2, h->nearest);
     k_props<<<grid_of(np, 256), 256, 0, s>>>(domain, sk, h->k2, h->k2 + np, h->nearest, nx, ny, resolution, mfp,
                                             locpore, kn, h->err);
     SH_TRY(hipGetLastError());
@@ -748,7 +751,6 @@ int mts_shape_run_static(int nx, int ny, const uint8_t* domain, double resolutio
     h.skel = base + L.skel;
     h.first = (int*)(base + L.first);
     h.last = (int*)(base + L.last);
-    h.g = (int*)(base + L.g);
     h.k2 = (int*)(base + L.k2);
     h.zrow = (int*)(base + L.zrow);
     h.nearest = (int*)(base + L.nearest);
