@@ -14,10 +14,10 @@
 //
 // Layout on the device: the canvas is bit-packed, one uint64 per 64 pixels
 // of a row (bit b = column 64 w + b), so that a thread evaluates the
-// deletion rule for 64 pixels with bitwise logic (bit-sliced counters for
+// deletion rule for 32 pixels with bitwise logic (bit-sliced counters for
 // the neighbour count and the 0->1 steps around the ring).  One launch runs
 // THIN_S subiterations of a 128 x 64-pixel tile in LDS (temporal blocking:
-// a halo of one word left and right and THIN_S rows above and below keeps
+// a halo of 32 pixels left and right and THIN_S rows above and below keeps
 // the inner tile exact).  Distances are exact integer squares: per-column
 // nearest zero (chunked scans), then the row minimum with early exit.
 #include <hip/hip_runtime.h>
