@@ -834,6 +834,7 @@ static int create_multi(mts_sim_s* s, int nx, int ny, const int32_t* pore, const
             (rc = upload(s->d_pixSite, site.data(), np * 4, s->stream)))
             return rc;
         HIP_TRY(hipStreamSynchronize(s->stream));  // the host maps go out of scope
+        if (np * 24 >= Readback::MIN_BYTES) (void)s->readback.ready();
     }
     upload_icsr(s->stream);
     upload_xynorm(s->stream);
@@ -1248,6 +1249,7 @@ int mts_create(int nx, int ny, const int32_t* pore, const double* kn, const doub
     upload_icsr(s->stream);
     upload_xynorm(s->stream);
     *out = s;
+    if ((size_t)s->P * 24 >= Readback::MIN_BYTES) (void)s->readback.ready();
     rc = mts_initialize(s);
     if (rc) {
         *out = nullptr;

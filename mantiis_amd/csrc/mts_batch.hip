@@ -645,6 +645,7 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
     b->active.assign(nb, 1);
     b->u_prev.assign(nb, 0.0);
     if ((rc = b->upload_queue())) return bail(rc);
+    if (*std::max_element(b->ncell.begin(), b->ncell.end()) * 12 >= (int64_t)Readback::SLOT) (void)b->readback.ready();
     if ((rc = b->step(true, 1))) return bail(rc);  // rest equilibrium -> first post-collision state
     e = hipStreamSynchronize(b->stream);
     if (e == hipSuccess) e = hipGetLastError();

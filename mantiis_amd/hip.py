@@ -242,7 +242,7 @@ class Lattice:
 
     def complete_domain(self):
         n = self.nx * self.ny
-        ux, uy, rho = np.empty(n), np.empty(n), np.empty(n)  # written whole
+        ux, uy, rho = np.zeros(n), np.zeros(n), np.zeros(n)
         _check(self.lib, self.lib.mts_complete_domain(self.h, _p(ux, _D), _p(uy, _D), _p(rho, _D)))
         return ux, uy, rho
 
