@@ -1244,6 +1244,7 @@ int mts_create(int nx, int ny, const int32_t* pore, const double* kn, const doub
         const float* cpar;
         if ((rc = upload_cpar(s, g.params, &cpar)) || (rc = upload_compact(s, s->cimg_h, cpar, s->cimg))) return bail(rc);
         upload_spec(s->cimg_h.spec, s->stream);
+        if ((rc = s->alloc(&s->cimg.X, (size_t)s->cimg_h.naux * 8))) return bail(rc);
         s->use_cimg = true;
     }
     upload_icsr(s->stream);

@@ -55,6 +55,8 @@ struct mts_batch_s {
     float* msnap = nullptr;
     int cur = 0;
     float* mac = nullptr;
+    float* xsnap = nullptr;  // the tuner's copy of the LINKS cells' side array
+    int64_t nside = 0;       // its size
     Readback readback;
     double* acc = nullptr;
     double* part = nullptr;      // per block
@@ -290,13 +292,20 @@ struct mts_batch_s {
         if (M[0] && !msnap) {
             if (int rc = alloc(&msnap, melems)) return rc;
         }
+        const size_t xelems = dev.X ? (size_t)nside : 0;
+        if (xelems && !xsnap) {
+            if (int rc = alloc(&xsnap, xelems)) return rc;
+        }
         BT_TRY(hipMemcpyAsync(snap, A[cur0], elems * sizeof(float), hipMemcpyDeviceToDevice, stream));
+        if (xelems) BT_TRY(hipMemcpyAsync(xsnap, dev.X, xelems * sizeof(float), hipMemcpyDeviceToDevice, stream));
         if (M[0]) BT_TRY(hipMemcpyAsync(msnap, M[cur0], melems * sizeof(float), hipMemcpyDeviceToDevice, stream));
         // puts the saved state back (also after a failed step: tuning never
         // leaves the batch partly advanced)
         auto restore = [&]() -> int {
             cur = cur0;
             if (hipMemcpyAsync(A[cur0], snap, elems * sizeof(float), hipMemcpyDeviceToDevice, stream) != hipSuccess ||
+                (xelems && hipMemcpyAsync(dev.X, xsnap, xelems * sizeof(float), hipMemcpyDeviceToDevice, stream) !=
+                               hipSuccess) ||
                 (M[0] && hipMemcpyAsync(M[cur0], msnap, melems * sizeof(float), hipMemcpyDeviceToDevice, stream) !=
                              hipSuccess) ||
                 hipStreamSynchronize(stream) != hipSuccess)
@@ -636,6 +645,8 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
     b->dev.ncell = base;
     b->dev.cstride = base;
     b->dev.inplace = !b->tiled && compact_inplace(C);
+    b->nside = C.naux * 8;
+    if (!b->tiled && b->nside && (rc = b->alloc(&b->dev.X, (size_t)b->nside))) return bail(rc);
     // drop the host copies of what now lives on the device
     C.cw = std::vector<uint32_t>();
     C.rw = std::vector<uint32_t>();

@@ -106,6 +106,11 @@ constexpr uint32_t CW_X_SHIFT = 25;
 // in link order when it is gathered (x-seam sites, buffer cells, irregular
 // wall links).  The others only take their sources from the record.
 constexpr uint32_t CW_RAW = CW_COMPLEX | CW_ISC_D;
+// Bit 24 marks a COMPLEX cell with two wall links of one specular slot, or one
+// whose specular slot streams: the pass that collides it adds its links up one
+// by one and keeps what goes to streaming slots in a side array (8 floats per
+// record), where there is one; otherwise it is treated as RAW.
+constexpr uint32_t CW_LINKS = CW_COMPLEX | CW_ISC_U;
 constexpr int CTILE_W = 128, CTILE_H = 8;  // Shan-Chen tile (sites)
 constexpr int CPAR_FLOATS = 12;  // FP32 parameter record of one (tau_s, Kn) pair
 constexpr int PLANE_GUARD = 64;  // elements after the last population plane (a neighbour index may be the cell count)

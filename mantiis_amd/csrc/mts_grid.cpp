@@ -335,18 +335,21 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
         }
         // A simple cell's slot j streams or is fed by its wall rule, and then
         // population opp(j) reaches no other cell: its plane holds the fed
-        // value between passes.  Its specular sources are those of its type
-        // (the kernels' table).  Cells that break this are RAW.
-        bool irregular = wall != 0 ? spec != ci.spec[t] : in != 0xffu;
+        // value between passes.  Cells that break this are RAW; cells whose
+        // specular links do not fit the kernels' table (one source for each fed
+        // slot of a type; about one cell in a million of a disk packing does
+        // not) are LINKS.
+        bool irregular = wall == 0 && in != 0xffu, links = wall != 0 && (ambiguous || spec != ci.spec[t]);
         for (int j = 1; wall != 0 && j < 9; j++) {
             const bool inj = (in >> (j - 1)) & 1u, fed = (wall >> (OPP[j] - 1)) & 1u;
-            if (inj == fed || (inj && ((spec >> (4 * (j - 1))) & 15u))) irregular = true;
+            if (inj == fed) irregular = true;
+            if (inj && ((spec >> (4 * (j - 1))) & 15u)) links = true;
             if (!((wall >> (j - 1)) & 1u)) continue;
             const int64_t q = (int64_t)wrap(y + EY[j], ny) * nx + wrap(x + EX[j], nx);
             if (ci.cidx[q] >= 0 && ((g.meta[q] >> (IN_SHIFT + j - 1)) & 1u)) irregular = true;
         }
-        const bool raw = irregular || (w & SEAM_BIT) || ambiguous || ovr >= 0;
-        const bool complex = raw || x == 0 || x == nx - 1 || (!g.torus && (y == 0 || y == ny - 1)) ||  // y-seam links lost
+        const bool raw = irregular || (w & SEAM_BIT) || ovr >= 0;
+        const bool complex = raw || links || x == 0 || x == nx - 1 || (!g.torus && (y == 0 || y == ny - 1)) ||  // y-seam links lost
                              p == g.gpIn || p == g.gpOut || ny < 3;
         auto push_aux = [&]() {  // explicit record of a COMPLEX cell
             const int32_t k = (int32_t)(ci.aux.size() / AUXW);
@@ -368,7 +371,7 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
         const int64_t du = (int64_t)rank[pu] - c, dd = c - (int64_t)rank[pd];
         const bool fits = du >= -32768 && du <= 32767 && dd >= -32768 && dd <= 32767;
         if (complex || !fits) {
-            cw = (cw & ~(CW_ISC_D | CW_ISC_U)) | (raw ? CW_RAW : CW_COMPLEX);
+            cw = (cw & ~(CW_ISC_D | CW_ISC_U)) | (raw ? CW_RAW : links ? CW_LINKS : CW_COMPLEX);
             ci.nraw += raw;
             ci.rw[c] = (uint32_t)push_aux();
         } else {

@@ -27,6 +27,7 @@ struct CompactDev {
     int64_t OS = 0;
     int ovr = 0;  // 0 gather, 1 take the override, 2 skip (see CImg)
     const float* M = nullptr;  // MDBB state read by the gather (set per launch)
+    float* X = nullptr;        // LINKS cells' side array: 8 floats per aux record (nullptr: they are RAW)
     bool inplace = false;      // steps may write where they read (no RAW cell, planes within 4 GiB)
 };
 

@@ -43,7 +43,7 @@ class Readback {
         size_t bytes;
     };
     static constexpr size_t SLOT = (size_t)1 << 20;  // bytes per thread: 8 MB pinned per handle (256 KB slots read at half the rate)
-    static constexpr size_t MIN_BYTES = (size_t)8 << 20;  // below, a plain copy costs less than pinning
+    static constexpr size_t MIN_BYTES = (size_t)24 << 20;  // below, a plain copy costs less than pinning
 
     // Pins the slots (a handle whose fields are large does so when it is made).
     bool ready() {

@@ -72,3 +72,56 @@ def test_fp32_transport_in_place(n, coll, wall, pairs, steps):
     o.run("transport", steps, 0.0)
     a, b = (np.asarray(x.get("f")).reshape(-1, 9) - w * rho0 for x in (g, o))
     assert rel_l2(a, b) <= 4 * 16 * 2.0**-24 * (2 * steps + 2)
+
+
+# a channel of two cells' width across a corner: two of its cells have wall
+# links whose specular slot streams, so their rule does not fit the per-type table
+DIAGONAL = """
+000001111111111
+000001111111111
+000001111111111
+000011111111111
+000011111110000
+000001111100000
+000000111000000
+000000011000000
+000000110000000
+000001111000000
+000011111000000
+000011111000000
+000001111110000
+000000111111111
+000000001111111
+"""
+
+
+@pytest.mark.parametrize("steps", [1, 2, 3, 6])
+@pytest.mark.parametrize("coll,wall", [(2, 2), (1, 2), (0, 2), (2, 0)])
+def test_fp32_links_cells(coll, wall, steps):
+    from mantiis_amd.hip import Batch
+    banner(f"FP32 transport with shared specular slots, collision {coll}, wall {wall}, {steps} steps")
+    pore = np.ones((48, 48), np.int32)
+    pore[16:31, 16:31] = np.array([[int(ch) for ch in row] for row in DIAGONAL.split()])
+    pore = np.ascontiguousarray(G.sanitize(pore), np.int32)
+    kn, lp = G.uniform_kn(pore, 0.1, MFP_DX)
+    par = dict(dx=1e-9, Fbody=1e-6)
+    o = O.Oracle(pore, kn, lp, periodic_y=True, **par)
+    o.set_operators(coll, wall)
+    o.run("transport", 40 + steps, 0.0)
+    g = Lattice(pore, kn, lp, precision="fp32dev", collision=coll, wall=wall, periodic_y=1, **par)
+    g.step("transport", 40)
+    g.step("transport", steps)
+    w = np.array([4 / 9] + [1 / 9] * 4 + [1 / 36] * 4)
+    rho0 = 0.235554544075989  # default gas state
+    a, b = (np.asarray(x.get("f")).reshape(-1, 9) - w * rho0 for x in (g, o))
+    assert rel_l2(a, b) <= 4 * 16 * 2.0**-24 * (40 + steps + 2)
+    # the batch (tuned: the tuner's steps must leave nothing behind)
+    bt = Batch([(pore, kn, lp)], collision=coll, wall=wall, **par)
+    bt.run(40, check_every=40, tol=1e-300)
+    bt.step(steps)
+    bt.run(2, check_every=2, tol=1e-300)
+    o = O.Oracle(pore, kn, lp, periodic_y=True, **par)
+    o.set_operators(coll, wall)
+    o.run("transport", 40 + steps + 2, 0.0)
+    for got, want in zip(bt.fields(0)[1:], o.complete_domain()[:2]):
+        assert rel_l2(np.asarray(got).reshape(-1), want) <= 4 * 16 * 2.0**-24 * (40 + steps + 3) * 10
