@@ -307,7 +307,8 @@ int mts_batch_step(mts_batch b, int nsteps);
  * the one-step cell-order kernel; *units = its tiles (32 x 16 sites) or
  * 256-cell blocks (either pointer may be NULL) */
 int mts_batch_kernel(mts_batch b, int* steps_per_launch, int64_t* units);
-/* marks lattices active (1) or not (0) for the next runs */
+/* marks lattices active (1) or not (0) for the next runs; an inactive lattice
+ * keeps its state, whatever the others run meanwhile */
 int mts_batch_activate(mts_batch b, const int32_t* active);
 /* rho, u_x, u_y (nx*ny row-major, solids 0) of lattice g's post-stream
  * state at the last check */

@@ -78,6 +78,7 @@ struct mts_batch_s {
     double* tpart = nullptr;  // per tile sums (zero for the tiles without a cell)
     int ntactive = 0;
     std::vector<char> active;
+    std::vector<signed char> home;  // per lattice outside the queue: the buffer of its state (-1: in the queue)
     std::vector<double> u_prev;
     std::vector<void*> allocs;
     // launch configuration of k_cbat (chosen by tune()): threads per
@@ -131,7 +132,28 @@ struct mts_batch_s {
         c.cimg = &dev;
         return c;
     }
+    // A lattice outside the queue keeps its state in the buffer that was current
+    // when it left; one that comes back after the buffers changed places is
+    // copied to the current one.
+    int settle() {
+        for (int g = 0; g < nb; g++) {
+            if (!active[g]) {
+                if (home[g] < 0) home[g] = (signed char)cur;
+                continue;
+            }
+            if (home[g] >= 0 && home[g] != cur) {
+                const size_t o = (size_t)off[g], n = (size_t)ncell[g] * sizeof(float), S = (size_t)dev.cstride;
+                for (int j = 0; j < 9; j++)
+                    BT_TRY(hipMemcpyAsync(A[cur] + j * S + o, A[cur ^ 1] + j * S + o, n, hipMemcpyDeviceToDevice, stream));
+                for (int j = 0; j < 4 && M[0]; j++)
+                    BT_TRY(hipMemcpyAsync(M[cur] + j * S + o, M[cur ^ 1] + j * S + o, n, hipMemcpyDeviceToDevice, stream));
+            }
+            home[g] = -1;
+        }
+        return MTS_OK;
+    }
     int upload_queue() {
+        if (int rc = settle()) return rc;
         // the active blocks' records in queue order, padded with empty
         // entries to the grid of a step
         std::vector<BatBlock> q;
@@ -217,7 +239,7 @@ struct mts_batch_s {
     // nsteps one-step launches, the last with statistics if asked for.  Pairs
     // run in place where the image allows it (an odd count starts with a step
     // to the other buffer, so the buffer changes as often as without pairs,
-    // modulo two, and lattices outside the queue are where they were)
+    // modulo two; see settle for the lattices outside the queue)
     int plain(int nsteps, bool stats) {
         int rc;
         const bool pairs = dev.inplace && prm.wall != MTS_WALL_MDBB;
@@ -654,6 +676,7 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
     C.outm = std::vector<uint8_t>();
     C.aux = std::vector<int32_t>();
     b->active.assign(nb, 1);
+    b->home.assign(nb, -1);
     b->u_prev.assign(nb, 0.0);
     if ((rc = b->upload_queue())) return bail(rc);
     if (*std::max_element(b->ncell.begin(), b->ncell.end()) * 12 >= (int64_t)Readback::SLOT) (void)b->readback.ready();
