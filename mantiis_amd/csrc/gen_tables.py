@@ -21,12 +21,12 @@ def main():
     out = ["// Generated by gen_tables.py from data/system_files -- do not edit.",
            "// 52 wall configurations of a cell's 3x3 neighbourhood (utils.hpp:728-793).",
            "#define MTS_NTYPES 52"]
-    out.append("static const int MTS_BND_CODE[52] = {" + ", ".join(str(v) for v in bt) + "};")
-    out.append("static const unsigned char MTS_IFSTREAM[52][9] = {" +
+    out.append("static constexpr int MTS_BND_CODE[52] = {" + ", ".join(str(v) for v in bt) + "};")
+    out.append("static constexpr unsigned char MTS_IFSTREAM[52][9] = {" +
                ", ".join("{" + ", ".join(str(v) for v in row) + "}" for row in ifs) + "};")
-    out.append("static const signed char MTS_ICSR[52][9] = {" +
+    out.append("static constexpr signed char MTS_ICSR[52][9] = {" +
                ", ".join("{" + ", ".join(str(v) for v in row) + "}" for row in icsr) + "};")
-    out.append("static const double MTS_XYNORM[52][2] = {" +
+    out.append("static constexpr double MTS_XYNORM[52][2] = {" +
                ", ".join("{%r, %r}" % (float(a), float(b)) for a, b in xy) + "};")
     with open(os.path.join(HERE, "mts_tables.inc"), "w") as f:
         f.write("\n".join(out) + "\n")

@@ -18,10 +18,6 @@
 #include "mts_readback.h"
 #include "mts_multigrid.h"
 
-namespace mts {
-void upload_xynorm(hipStream_t st);
-}
-
 using namespace mts;
 
 static thread_local std::string g_err;
@@ -673,7 +669,6 @@ static int create_multi32(mts_sim_s* s, const std::vector<CoarseRow>& cr, const 
         C.ovr = C.plain;
         C.ovr.ovr = 1;
     }
-    upload_spec(s->lc[0].h.spec, s->stream);
     // interface plans of the pairs, in cell indices with host-formed weights
     IfPlan all;
     s->ifb_off.assign(1, 0);
@@ -836,8 +831,6 @@ static int create_multi(mts_sim_s* s, int nx, int ny, const int32_t* pore, const
         HIP_TRY(hipStreamSynchronize(s->stream));  // the host maps go out of scope
         if (np * 24 >= Readback::MIN_BYTES) (void)s->readback.ready();
     }
-    upload_icsr(s->stream);
-    upload_xynorm(s->stream);
     for (size_t l = 0; l < s->lv.size(); l++) {
         LaunchCtx c = s->lctx((int)l);
         launch_init(c, s->lv[l].d_f);
@@ -1243,12 +1236,9 @@ int mts_create(int nx, int ny, const int32_t* pore, const double* kn, const doub
     if (fp32) {
         const float* cpar;
         if ((rc = upload_cpar(s, g.params, &cpar)) || (rc = upload_compact(s, s->cimg_h, cpar, s->cimg))) return bail(rc);
-        upload_spec(s->cimg_h.spec, s->stream);
         if ((rc = s->alloc(&s->cimg.X, (size_t)s->cimg_h.naux * 8))) return bail(rc);
         s->use_cimg = true;
     }
-    upload_icsr(s->stream);
-    upload_xynorm(s->stream);
     *out = s;
     if ((size_t)s->P * 24 >= Readback::MIN_BYTES) (void)s->readback.ready();
     rc = mts_initialize(s);

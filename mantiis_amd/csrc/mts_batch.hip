@@ -587,7 +587,6 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
         C.rw.resize(base, 0u);
         C.pidx.resize(base, 0);
         C.outm.resize(base, 0);
-        if (g == 0) canonical_spec(C.spec);
         B = Built();  // release the lattice's host tables
     }
     b->tfirst[nb] = b->ntiles;
@@ -655,8 +654,6 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
     }
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
     if (e != hipSuccess) return bail(set_error(MTS_ERR_HIP, std::string("upload: ") + hipGetErrorString(e)));
-    upload_spec(C.spec, b->stream);
-    upload_icsr(b->stream);
     b->dev.cw = cw;
     b->dev.rw = rw;
     b->dev.pidx = pidx;

@@ -128,13 +128,7 @@ struct CompactImage {
     std::vector<int32_t> cidx;     // [nx*ny] site -> cell or -1
     std::vector<int32_t> cellPos;  // [ncell] cell -> site
     std::vector<int32_t> segs;     // [ny * (ntx+1)]: cells before the site (tx*CTILE_W, y)
-    uint32_t spec[64] = {};        // per TYPE: slot j's specular source ic in bits 4(j-1)..4j-1
 };
-
-// The specular-source table of the cell-order kernels (the same for every
-// lattice): per boundary type (52 = typeless, full bounce-back), slot j's
-// source link ic, taken when ic is a wall link of the cell.
-void canonical_spec(uint32_t spec[64]);
 
 // A site image to put in cell order: link words and parameter indices per
 // site, the generalized-periodic sites and, per site, the slot of an

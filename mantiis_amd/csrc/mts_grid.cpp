@@ -10,7 +10,7 @@
 
 #include "mantiis_hip.h"
 #include "mts_common.h"
-#include "mts_tables.inc"
+#include "mts_consttab.h"
 
 namespace mts {
 
@@ -257,19 +257,6 @@ void decode_links(const Geometry& g, int which, std::vector<int64_t>& id, std::v
     }
 }
 
-void canonical_spec(uint32_t spec[64]) {
-    // slot j <- the link ic that is not streamed for the type and whose
-    // specular direction is j (the first such link when two share a slot)
-    for (int t = 0; t < 64; t++) spec[t] = 0;
-    for (int t = 0; t <= MTS_NTYPES; t++)
-        for (int ic = 8; ic >= 1; ic--) {
-            const bool wl = t == MTS_NTYPES ? true : !MTS_IFSTREAM[t][ic];
-            const int sr = t == MTS_NTYPES ? OPP[ic] : MTS_ICSR[t][ic];
-            if (!wl || sr <= 0) continue;
-            spec[t] = (spec[t] & ~(15u << (4 * (sr - 1)))) | ((uint32_t)ic << (4 * (sr - 1)));
-        }
-}
-
 void build_compact(const Geometry& g, CompactImage& ci) {
     LatticeView v{g.nx, g.ny, g.torus, g.meta.data(), g.pidx.data(), g.gpIn, g.gpOut, nullptr};
     build_compact(v, ci);
@@ -310,7 +297,7 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
     ci.outm.assign(n, 0);
     ci.aux.clear();
     ci.nraw = 0;
-    canonical_spec(ci.spec);
+    static constexpr TypeWords SPEC = spec_words();  // the kernels' table
     for (int64_t c = 0; c < n; c++) {
         const int64_t p = ci.cellPos[c];
         const int x = (int)(p % nx), y = (int)(p / nx);
@@ -339,7 +326,7 @@ void build_compact(const LatticeView& g, CompactImage& ci) {
         // specular links do not fit the kernels' table (one source for each fed
         // slot of a type; about one cell in a million of a disk packing does
         // not) are LINKS.
-        bool irregular = wall == 0 && in != 0xffu, links = wall != 0 && (ambiguous || spec != ci.spec[t]);
+        bool irregular = wall == 0 && in != 0xffu, links = wall != 0 && (ambiguous || spec != SPEC[t]);
         for (int j = 1; wall != 0 && j < 9; j++) {
             const bool inj = (in >> (j - 1)) & 1u, fed = (wall >> (OPP[j] - 1)) & 1u;
             if (inj == fed) irregular = true;

@@ -145,9 +145,7 @@ struct IfSpec {
 int launch_cinterface_step(const LaunchCtx& c1, const MbSpec& s1, const LaunchCtx& c2, const MbSpec& s2,
                            const IfSpec& f);
 
-void upload_icsr(hipStream_t st);
 // FP32 production kernels in cell order (mts_compact.inc)
-void upload_spec(const uint32_t* spec64, hipStream_t st);
 // The FP32 parameter records (8 floats per (tau_s, Kn) pair) and the SRBB
 // bookkeeping table (24 floats per pair) of a parameter list.
 void fp32_params(const std::vector<CellParam>& params, double rho0, std::vector<float>& cpar, std::vector<float>& book);

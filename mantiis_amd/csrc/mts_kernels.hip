@@ -25,7 +25,7 @@
 
 #include "mts_common.h"
 #include "mts_kernels.h"
-#include "mts_tables.inc"
+#include "mts_consttab.h"
 
 namespace mts {
 namespace dev {
@@ -68,12 +68,9 @@ __device__ __forceinline__ constexpr double Mi(int k, int v) {
     return MI[k * 9 + v];
 }
 
-// icsr table (utils.hpp:749-767), 0-based; row MTS_NTYPES is the typeless
-// wall link of a buffer cell (full bounce-back: target = opposite).
-__constant__ signed char c_icsr[MTS_NTYPES + 1][9];
-// the same for ic = 1..8 in bits 4(ic-1)..4ic-1 of one word per type
-// (TYPE_NONE takes the typeless row; its sites have no wall link)
-__constant__ uint32_t c_icsr4[64];
+// specular targets per boundary type, as a table and as one word per type
+__constant__ IcsrTable c_icsr = icsr_table();
+__constant__ TypeWords c_icsr4 = icsr_words();
 
 // Site helpers ---------------------------------------------------------------
 struct Lat {
@@ -263,7 +260,7 @@ __device__ __forceinline__ void gather(const double* __restrict__ A, const Lat& 
     if (wall) {
 #pragma unroll
         for (int j = 1; j < 9; j++) own[j] = ld64(A, (int64_t)j * L.stride + p);
-        if (WALL != MTS_WALL_BB) spec = c_icsr4[(w >> TYPE_SHIFT) & 63u];
+        if (WALL != MTS_WALL_BB) spec = c_icsr4.v[(w >> TYPE_SHIFT) & 63u];
     } else {
 #pragma unroll
         for (int j = 1; j < 9; j++) own[j] = 0.0;
@@ -676,20 +673,6 @@ template <typename K, typename... A>
 static void klaunch(K k, dim3 g, dim3 b, uint32_t sh, const LaunchCtx& c, A... a) {
     if (c.ev0) hipExtLaunchKernelGGL(k, g, b, sh, c.stream, c.ev0, c.ev1, 0, a...);
     else hipLaunchKernelGGL(k, g, b, sh, c.stream, a...);
-}
-
-void upload_icsr(hipStream_t st) {
-    signed char t[MTS_NTYPES + 1][9];
-    for (int i = 0; i < MTS_NTYPES; i++)
-        for (int j = 0; j < 9; j++) t[i][j] = MTS_ICSR[i][j] < 0 ? 0 : MTS_ICSR[i][j];
-    for (int j = 0; j < 9; j++) t[MTS_NTYPES][j] = (signed char)OPP[j];
-    static uint32_t t4[64];
-    for (int i = 0; i < 64; i++) {
-        t4[i] = 0;
-        for (int j = 1; j < 9; j++) t4[i] |= (uint32_t)t[i < MTS_NTYPES ? i : MTS_NTYPES][j] << (4 * (j - 1));
-    }
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_icsr4), t4, sizeof(t4), 0, hipMemcpyHostToDevice, st);
-    (void)hipMemcpyToSymbolAsync(HIP_SYMBOL(c_icsr), t, sizeof(t), 0, hipMemcpyHostToDevice, st);
 }
 
 template <int MODE, int COLL, int WALL>
