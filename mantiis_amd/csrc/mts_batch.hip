@@ -367,9 +367,12 @@ struct mts_batch_s {
         }
         // the short timings do not separate the queue maps of one launch width
         // within about 1%: of those that close to the fastest, take the
-        // longest XCD run (the fewest bytes fetched from memory)
+        // longest XCD run (the fewest bytes fetched from memory).  Populations
+        // that stay in the 256 MB Infinity Cache are fetched from there whatever
+        // the map, and the fastest is taken as timed.
         const int b0 = best;
-        for (int k = 0; k < NCAND; k++)
+        const bool cached = elems * sizeof(float) <= (size_t)256 << 20;
+        for (int k = 0; k < NCAND && !cached; k++)
             if (tune_ms[k] > 0.0 && cand_threads(k) == cand_threads(b0) && cand_xrun(k) > cand_xrun(best) &&
                 tune_ms[k] <= 1.01 * tune_ms[b0])
                 best = k;
