@@ -34,6 +34,13 @@ int set_error(int code, const std::string& msg);  // mts_api.hip
                              std::string(#expr) + ": " + hipGetErrorString(e_));           \
     } while (0)
 
+// Cells from which mts_batch_fields reads a lattice through the pinned slots.
+// Below, starting the threads costs more than they save: microseconds per
+// lattice, one copy against slots, porosity 0.6: 400^2 (96,000 cells) 177 / 248,
+// 512^2 (157,000) 264 / 358, 560^2 (188,000) 353 / 424, 600^2 (216,000) 441-533 /
+// 464-478, 640^2 (246,000) 541 / 512, 700^2 (294,000) 776 / 584, 1024^2 1780 / 1150.
+constexpr size_t FIELDS_PINNED = 220000;
+
 struct mts_batch_s {
     mts_params prm{};
     Physics ph;
@@ -679,7 +686,7 @@ int mts_batch_create(int nb, const int* nx, const int* ny, const int32_t* const*
     b->home.assign(nb, -1);
     b->u_prev.assign(nb, 0.0);
     if ((rc = b->upload_queue())) return bail(rc);
-    if (*std::max_element(b->ncell.begin(), b->ncell.end()) * 12 >= (int64_t)Readback::SLOT) (void)b->readback.ready();
+    if ((size_t)*std::max_element(b->ncell.begin(), b->ncell.end()) >= FIELDS_PINNED) (void)b->readback.ready();
     if ((rc = b->step(true, 1))) return bail(rc);  // rest equilibrium -> first post-collision state
     e = hipStreamSynchronize(b->stream);
     if (e == hipSuccess) e = hipGetLastError();
@@ -844,7 +851,7 @@ int mts_batch_fields(mts_batch b, int g, double* rho, double* ux, double* uy) {
         }
         return hipSuccess;
     };
-    if ((size_t)n * 12 >= Readback::SLOT && b->readback.ready()) {
+    if ((size_t)n >= FIELDS_PINNED && b->readback.ready()) {
         const int64_t per = (int64_t)(Readback::SLOT / 4 / 12) / 64 * 64;  // a quarter slot: work for every thread
         BT_TRY(b->readback.each(b->prm.device, b->stream, (size_t)((n + per - 1) / per),
                                 [&](size_t i, char* slot) { return fetch((float*)slot, i * per, std::min<int64_t>(n, (i + 1) * per)); },
