@@ -216,7 +216,6 @@ struct ConvArgs {
     int Cin, Cout, ksz, sgn;  // sgn: +1 forward, -1 backward data (offsets reversed)
     int steps;                // products of 32 deep: ceil(ksz^2 Cin / 32)
     int tilesX, tilesY;
-    int direct;               // the tile does not fit in LDS: operands come from memory
     const bf16* Wf;           // packed weights (k_pack)
     const float* bias;        // forward
     const bf16* mask;         // backward, BF16 output: the ReLU output whose gradient this is
@@ -250,7 +249,8 @@ inline size_t conv_lds(int Cin, int ksz, int steps, int rows) {
 // fetched every input element nine times through per-element index divisions,
 // took 1703 us; a training step on eight 256 x 256 images went from 5.02 to
 // 2.08 ms with k_convw.
-template <int MTW, int NTW, int WM, int WN>
+// MEM: operands from memory, for tiles that do not fit in LDS.
+template <int MTW, int NTW, int WM, int WN, bool MEM>
 __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
     extern __shared__ char lds[];
     constexpr int TH = WM * MTW, CH = WN * NTW;
@@ -266,7 +266,7 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
     int* s_off = (int*)lds;
     char* tile = lds + conv_off_bytes(a.steps, small);
     const int ng = a.ksz * a.ksz * (small ? a.Cin : C8);
-    if (!a.direct) {
+    if (!MEM) {
         for (int g = t; g < (small ? 32 : a.steps * 4); g += 256) {
             const int d = small ? a.Cin : C8, kk = g / d, c = g - kk * d;
             int dy, dx;
@@ -307,7 +307,7 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
     // weights of step k: CH tiles of 64 lanes x 8 elements
     const bf16x8* wp = (const bf16x8*)a.Wf + ((int64_t)blockIdx.y * a.steps * CH + wn * NTW) * 64 + l;
     const char* px0 = tile + ((wm * MTW) * LW + i) * PS;
-    if (!a.direct && !small) {
+    if (!MEM && !small) {
         // Weights and offsets are read two steps ahead and pixels one, so that
         // a step's products wait for nothing they have just asked for; the
         // rings' places are fixed by unrolling six steps.
@@ -350,35 +350,60 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
                         acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u % 3][n], xf[u % 2][m], acc[m][n], 0, 0, 0);
             }
         }
-    } else {
+    } else if (!MEM) {
         __syncthreads();
         for (int k = 0; k < a.steps; k++) {
             bf16x8 xf[MTW];
-            if (small) {
 #pragma unroll
-                for (int m = 0; m < MTW; m++)
+            for (int m = 0; m < MTW; m++)
 #pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const bf16 v = *(const bf16*)(px0 + m * LW * PS + s_off[8 * q + e]);
-                        xf[m][e] = 8 * q + e < ng ? v : (bf16)0.0f;
-                    }
-            } else {
-                const int g = 4 * k + q, kk = min(g / C8, a.ksz * a.ksz - 1), c8 = g - g / C8 * C8;
-                int dy, dx;
-                koff(kk, a.ksz, dy, dx);
-#pragma unroll
-                for (int m = 0; m < MTW; m++) {
-                    const bf16x8 v = *(const bf16x8*)a.in.at(b, wrapn(y0 + wm * MTW + m + a.sgn * dy, H),
-                                                             wrapn(x0 + i + a.sgn * dx, W), c8 * 8);
-                    xf[m] = g < ng ? v : bf16x8{};
+                for (int e = 0; e < 8; e++) {
+                    const bf16 v = *(const bf16*)(px0 + m * LW * PS + s_off[8 * q + e]);
+                    xf[m][e] = 8 * q + e < ng ? v : (bf16)0.0f;
                 }
-            }
 #pragma unroll
             for (int n = 0; n < NTW; n++) {
                 const bf16x8 wv = wp[(k * CH + n) * 64];
 #pragma unroll
                 for (int m = 0; m < MTW; m++)
                     acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, xf[m], acc[m][n], 0, 0, 0);
+            }
+        }
+    } else {
+        // A step's operands are read AHEAD steps before its products: reading
+        // them when they are used made every step a round trip to memory (one
+        // 128 x 128 image, 96 base channels: 912 us, 614 so, 831 in the former
+        // implicit GEMM).
+        constexpr int AHEAD = 4;
+        bf16x8 wr[AHEAD][NTW], xf[AHEAD][MTW];
+        auto fetch = [&](int k, bf16x8* wv, bf16x8* xv) {
+            const int g = 4 * k + q, kk = min(g / C8, a.ksz * a.ksz - 1), c8 = g - g / C8 * C8;
+            int dy, dx;
+            koff(kk, a.ksz, dy, dx);
+#pragma unroll
+            for (int n = 0; n < NTW; n++) wv[n] = wp[(k * CH + n) * 64];
+#pragma unroll
+            for (int m = 0; m < MTW; m++)
+                xv[m] = *(const bf16x8*)a.in.at(b, wrapn(y0 + wm * MTW + m + a.sgn * dy, H), wrapn(x0 + i + a.sgn * dx, W),
+                                                c8 * 8);
+        };
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++)
+            if (u < a.steps) fetch(u, wr[u], xf[u]);
+        for (int k0 = 0; k0 < a.steps; k0 += AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) {
+                const int k = k0 + u;
+                if (k >= a.steps) break;
+                if (4 * k + 3 >= ng && 4 * k + q >= ng)  // past the last group (see above)
+#pragma unroll
+                    for (int m = 0; m < MTW; m++) xf[u][m] = bf16x8{};
+#pragma unroll
+                for (int n = 0; n < NTW; n++)
+#pragma unroll
+                    for (int m = 0; m < MTW; m++)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[u][n], xf[u][m], acc[m][n], 0, 0, 0);
+                if (k + AHEAD < a.steps) fetch(k + AHEAD, wr[u], xf[u]);
             }
         }
     }
@@ -475,16 +500,16 @@ inline int64_t conv_pack_elems(int Cin, int Cout, int ksz) {
     return (int64_t)conv_chunks(Cout) * conv_steps(Cin, ksz) * conv_chunk(Cout) * 512;
 }
 
-template <int MTW, int NTW, int WM, int WN>
+template <int MTW, int NTW, int WM, int WN, bool MEM = false>
 int launch_conv_t(ConvArgs& a, int B, size_t lds, hipStream_t st) {
     a.tilesX = (a.in.W + 15) / 16;
     a.tilesY = (a.in.H + WM * MTW - 1) / (WM * MTW);
     if (lds > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k_conv<MTW, NTW, WM, WN>,
+        const hipError_t e = hipFuncSetAttribute((const void*)k_conv<MTW, NTW, WM, WN, MEM>,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
     }
-    hipLaunchKernelGGL((k_conv<MTW, NTW, WM, WN>), dim3(a.tilesX * a.tilesY * B, conv_chunks(a.Cout)), dim3(256), lds, st, a);
+    hipLaunchKernelGGL((k_conv<MTW, NTW, WM, WN, MEM>), dim3(a.tilesX * a.tilesY * B, conv_chunks(a.Cout)), dim3(256), lds, st, a);
     return 0;
 }
 
@@ -498,9 +523,14 @@ inline int launch_conv(ConvArgs a, int B, hipStream_t st) {
         return (int64_t)((a.in.W + 15) / 16) * ((a.in.H + r - 1) / r) * B * conv_chunks(a.Cout);
     };
     while (rows > 4 && (conv_lds(a.Cin, a.ksz, a.steps, rows) > CU_LDS / 2 || blocks(rows) < 512)) rows /= 2;
-    size_t lds = conv_lds(a.Cin, a.ksz, a.steps, rows);
-    a.direct = lds > CU_LDS;
-    if (a.direct) lds = 0;
+    const size_t lds = conv_lds(a.Cin, a.ksz, a.steps, rows);
+    if (lds > CU_LDS) switch (conv_chunk(a.Cout)) {
+        case 1: return launch_conv_t<1, 1, 4, 1, true>(a, B, 0, st);
+        case 2: return launch_conv_t<1, 2, 4, 1, true>(a, B, 0, st);
+        case 3: return launch_conv_t<1, 3, 4, 1, true>(a, B, 0, st);
+        case 4: return launch_conv_t<2, 2, 2, 2, true>(a, B, 0, st);
+        default: return launch_conv_t<2, 3, 2, 2, true>(a, B, 0, st);
+    }
     switch (conv_chunk(a.Cout) * 100 + rows) {
         case 116: return launch_conv_t<4, 1, 4, 1>(a, B, lds, st);
         case 108: return launch_conv_t<2, 1, 4, 1>(a, B, lds, st);
