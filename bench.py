@@ -512,7 +512,7 @@ def bench_warmstart(args):
                                f"({args.epochs} epochs, U-Net c0={c0}, {len(params)} parameters), infer {args.eval} "
                                "unseen 512^2 lattices, then LBM to |d<u_x>/dt|/|<u_x>| < 1e-6 per step",
                    "parallelism": "single GPU"},
-        "roofline": {"bound": "mfma", "kernel": "k_gemm (BF16 MFMA implicit GEMM, training step)",
+        "roofline": {"bound": "mfma", "kernel": "k_conv, k_convw (BF16 MFMA convolutions, training step)",
                      "achieved": round(tflops, 2), "peak": 2500.0, "unit": "TFLOP/s", "frac": round(tflops / 2500.0, 5),
                      "traffic": None},
         "cpu_baseline": None,

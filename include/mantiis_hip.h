@@ -372,8 +372,9 @@ int mts_net_forward(mts_net n, const float* in, int B, int H, int W, float* out)
  * and the gradient of every parameter */
 int mts_net_backward(mts_net n, const float* target, const float* mask, float* loss);
 int mts_net_adam(mts_net n, float lr, float beta1, float beta2, float eps, int step);
-/* the convolutions' GEMM kernel on dense host matrices (check of the matrix
- * core lane layout): C[M x N] = A[M x K] B[K x N] with BF16 operands */
+/* the convolution kernel on dense host matrices, as a 1x1 convolution of M
+ * pixels (check of the matrix core lane layout): C[M x N] = A[M x K] B[K x N]
+ * with BF16 operands */
 int mts_net_gemm_check(const float* A, const float* B, int M, int N, int K, float* C);
 int mts_net_stream(mts_net n, void** stream);
 

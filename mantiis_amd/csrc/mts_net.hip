@@ -46,143 +46,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int TM = 64, TN = 64, TK = 64, LDK = TK + 8;
-
-// ---------------------------------------------------------------- GEMM
-// C[M x N] = A[M x K] B[K x N] on dense operands (mts_net_gemm_check).
-// Lane layout of v_mfma_f32_16x16x32_bf16 (wave64): lane l holds
-// A[l % 16][8 (l / 16) .. +7], B[8 (l / 16) .. +7][l % 16] and
-// D[4 (l / 16) .. +3][l % 16].
-// A stage is TK = 64 deep: each thread holds two 8-element fragments of A and
-// of B in registers.  The next stage's fragments are loaded from memory
-// before the current stage's eight MFMAs per wave, and written to LDS after
-// them, so the loads overlap the matrix work.
 typedef uint4 v16;
-struct Frag {
-    v16 v;
-};
-
-template <class Op>
-__global__ void __launch_bounds__(256) k_gemm(Op op, int M, int N, int K, int nsplit, int kchunk) {
-    __shared__ bf16 sA[TM][LDK];
-    __shared__ bf16 sB[TN][LDK];
-    const int m0 = blockIdx.x * TM, n0 = blockIdx.y * TN, z = blockIdx.z;
-    const int kb = (z % nsplit) * kchunk, ke = min(K, kb + kchunk);
-    const int t = threadIdx.x, w = t >> 6, l = t & 63;
-    const int wm = (w & 1) * 32, wn = (w >> 1) * 32;
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    Frag fa[2], fb[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        op.load_a(fa[h], m0, kb, ke, M, z, t, h);
-        op.load_b(fb[h], n0, kb, ke, N, z, t, h);
-    }
-    for (int k0 = kb; k0 < ke; k0 += TK) {
-        op.store_a(sA, fa, t);
-        op.store_b(sB, fb, t);
-        __syncthreads();
-        if (k0 + TK < ke) {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                op.load_a(fa[h], m0, k0 + TK, ke, M, z, t, h);
-                op.load_b(fb[h], n0, k0 + TK, ke, N, z, t, h);
-            }
-        }
-        const int i = l & 15, q = (l >> 4) * 8;
-#pragma unroll
-        for (int kh = 0; kh < 2; kh++) {
-            bf16x8 af[2], bfm[2];
-#pragma unroll
-            for (int a = 0; a < 2; a++) af[a] = *(const bf16x8*)&sA[wm + a * 16 + i][32 * kh + q];
-#pragma unroll
-            for (int b = 0; b < 2; b++) bfm[b] = *(const bf16x8*)&sB[wn + b * 16 + i][32 * kh + q];
-#pragma unroll
-            for (int a = 0; a < 2; a++)
-#pragma unroll
-                for (int b = 0; b < 2; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfm[b], acc[a][b], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int rr = 0; rr < 4; rr++) {
-                const int m = m0 + wm + a * 16 + 4 * (l >> 4) + rr, n = n0 + wn + b * 16 + (l & 15);
-                if (m < M && n < N) op.store(m, n, acc[a][b][rr], z);
-            }
-}
-
-// Fragment loads and LDS stores.  Row layout: thread t takes tile row t/4
-// and the 8 consecutive k from 8 (t%4) + 32 h; one 16-byte load when the
-// operand keeps those 8 k contiguous (pa/pb), element loads otherwise.
-// Transposed layout (operands whose 8 contiguous elements run along the
-// tile's row index, e.g. 8 channels of one pixel): thread t takes rows
-// 8 (t%8) .. +7 at k = 2 (t/8) + h, so its two fragments fill 4-byte pairs.
-__device__ __forceinline__ void row_store(bf16 (*s)[LDK], const Frag* f, int t) {
-#pragma unroll
-    for (int h = 0; h < 2; h++) *(v16*)&s[t >> 2][(t & 3) * 8 + 32 * h] = f[h].v;
-}
-__device__ __forceinline__ void tr_store(bf16 (*s)[LDK], const Frag* f, int t) {
-    const uint16_t* a = (const uint16_t*)&f[0].v;
-    const uint16_t* b = (const uint16_t*)&f[1].v;
-    const int gq = (t & 7) * 8, p = 2 * (t >> 3);
-#pragma unroll
-    for (int e = 0; e < 8; e++) *(uint32_t*)&s[gq + e][p] = (uint32_t)a[e] | ((uint32_t)b[e] << 16);
-}
-template <class Op>
-__device__ __forceinline__ void row_load_a(const Op& op, Frag& f, int m0, int k0, int ke, int M, int z, int t, int h) {
-    const int m = m0 + (t >> 2), k = k0 + (t & 3) * 8 + 32 * h;
-    if (op.vec_a && m < M && k + 7 < ke) {
-        f.v = *(const v16*)op.pa(m, k, z);
-        return;
-    }
-    bf16* e8 = (bf16*)&f.v;
-#pragma unroll
-    for (int e = 0; e < 8; e++) e8[e] = (m < M && k + e < ke) ? op.a(m, k + e, z) : (bf16)0.0f;
-}
-template <class Op>
-__device__ __forceinline__ void row_load_b(const Op& op, Frag& f, int n0, int k0, int ke, int N, int z, int t, int h) {
-    const int n = n0 + (t >> 2), k = k0 + (t & 3) * 8 + 32 * h;
-    if (op.vec_b && n < N && k + 7 < ke) {
-        f.v = *(const v16*)op.pb(k, n, z);
-        return;
-    }
-    bf16* e8 = (bf16*)&f.v;
-#pragma unroll
-    for (int e = 0; e < 8; e++) e8[e] = (n < N && k + e < ke) ? op.b(k + e, n, z) : (bf16)0.0f;
-}
-
-// row-layout operands (dense and convolution forward / backward-data)
-#define MTS_ROW_FILLS                                                                                       \
-    __device__ void load_a(Frag& f, int m0, int k0, int ke, int M, int z, int t, int h) const {             \
-        row_load_a(*this, f, m0, k0, ke, M, z, t, h);                                                       \
-    }                                                                                                       \
-    __device__ void load_b(Frag& f, int n0, int k0, int ke, int N, int z, int t, int h) const {             \
-        row_load_b(*this, f, n0, k0, ke, N, z, t, h);                                                       \
-    }                                                                                                       \
-    __device__ void store_a(bf16 (*s)[LDK], const Frag* f, int t) const { row_store(s, f, t); }             \
-    __device__ void store_b(bf16 (*s)[LDK], const Frag* f, int t) const { row_store(s, f, t); }
-
-// dense row-major operands (the GEMM check)
-struct OpDense {
-    const bf16 *A, *B;
-    float* C;
-    int K, N;
-    static constexpr bool vec_a = false, vec_b = false;
-    __device__ bf16 a(int m, int k, int) const { return A[(int64_t)m * K + k]; }
-    __device__ bf16 b(int k, int n, int) const { return B[(int64_t)k * N + n]; }
-    __device__ const bf16* pa(int, int, int) const { return nullptr; }
-    __device__ const bf16* pb(int, int, int) const { return nullptr; }
-    MTS_ROW_FILLS
-    __device__ void store(int m, int n, float v, int) const { C[(int64_t)m * N + n] = v; }
-};
 
 // ---------------------------------------------------------------- convolution
 __device__ __forceinline__ int wrapn(int v, int n) {  // v >= -n
@@ -416,9 +280,9 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
     for (int n = 0; n < NTW; n++) {
         const int c = ((blockIdx.y * WN + wn) * NTW + n) * 16 + 4 * q;
         if (c >= a.Cout) continue;
-        if (a.Cout & 3) {  // the head's two channels
+        if (a.Cout & 3) {  // the head's two channels, odd widths of the check
             for (int m = 0; m < MTW && y1 + m < H; m++)
-                for (int e = 0; e < a.Cout - c; e++) {
+                for (int e = 0; e < min(4, a.Cout - c); e++) {
                     const int64_t o = o0 + (int64_t)m * rowStep + c + e;
                     float v = acc[0][n][e];
 #pragma unroll
@@ -959,12 +823,6 @@ __global__ void k_adam(float* w, const float* g, float* m, float* v, int64_t n, 
 
 inline unsigned nblk(int64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
-template <class Op>
-void gemm(const Op& op, int M, int N, int K, int nz, int nsplit, int kchunk, hipStream_t st) {
-    dim3 grid((M + TM - 1) / TM, (N + TN - 1) / TN, nz);
-    hipLaunchKernelGGL(k_gemm<Op>, grid, dim3(256), 0, st, op, M, N, K, nsplit, kchunk);
-}
-
 }  // namespace net
 
 using namespace net;
@@ -1377,32 +1235,51 @@ int mts_net_adam(mts_net n, float lr, float beta1, float beta2, float eps, int s
     return MTS_OK;
 }
 
-// The GEMM kernel on dense host matrices (A: M x K, B: K x N, row-major,
-// rounded to BF16 on the device): C = A B in FP32.
+// C = A B on dense host matrices (A: M x K, B: K x N, row-major, rounded to
+// BF16 on the device) as the layers compute it: a 1x1 convolution of M pixels
+// with K input and N output channels (K padded with zeros to whole vectors).
 int mts_net_gemm_check(const float* A, const float* Bm, int M, int N, int K, float* C) {
     if (!A || !Bm || !C || M <= 0 || N <= 0 || K <= 0 || (int64_t)M * N > (1 << 24) || (int64_t)M * K > (1 << 24) ||
         (int64_t)K * N > (1 << 24))
         return set_error(MTS_ERR_ARG, "bad GEMM check shape");
-    float *dA, *dB, *dC;
-    bf16 *hA, *hB;
-    NET_TRY(hipMalloc(&dA, (size_t)M * K * 4));
-    NET_TRY(hipMalloc(&dB, (size_t)K * N * 4));
-    NET_TRY(hipMalloc(&dC, (size_t)M * N * 4));
-    NET_TRY(hipMalloc(&hA, (size_t)M * K * 2));
-    NET_TRY(hipMalloc(&hB, (size_t)K * N * 2));
-    NET_TRY(hipMemcpy(dA, A, (size_t)M * K * 4, hipMemcpyHostToDevice));
-    NET_TRY(hipMemcpy(dB, Bm, (size_t)K * N * 4, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_f2bf, dim3(nblk((int64_t)M * K)), dim3(256), 0, nullptr, dA, hA, (int64_t)M * K);
-    hipLaunchKernelGGL(k_f2bf, dim3(nblk((int64_t)K * N)), dim3(256), 0, nullptr, dB, hB, (int64_t)K * N);
-    OpDense op{hA, hB, dC, K, N};
-    gemm(op, M, N, K, 1, 1, K, nullptr);
+    const int Kp = (K + 7) / 8 * 8;
+    std::vector<float> a, w;  // A padded; B as weights [N][Kp]
+    try {
+        a.assign((size_t)M * Kp, 0.0f);
+        w.assign((size_t)N * Kp, 0.0f);
+    } catch (...) {
+        return set_error(MTS_ERR_OOM, "host allocation");
+    }
+    for (int m = 0; m < M; m++) std::copy(A + (size_t)m * K, A + (size_t)(m + 1) * K, &a[(size_t)m * Kp]);
+    for (int k = 0; k < K; k++)
+        for (int n = 0; n < N; n++) w[(size_t)n * Kp + k] = Bm[(size_t)k * N + n];
+    mts_net_s d;  // owns the buffers and the stream
+    float *dA, *dW, *dC;
+    bf16 *hA, *hW;
+    NET_TRY(hipStreamCreateWithFlags(&d.stream, hipStreamNonBlocking));
+    const int64_t nw = conv_pack_elems(Kp, N, 1);
+    int rc;
+    if ((rc = d.alloc(&dA, a.size())) || (rc = d.alloc(&dW, w.size())) || (rc = d.alloc(&dC, (size_t)M * N)) ||
+        (rc = d.alloc(&hA, a.size())) || (rc = d.alloc(&hW, nw)))
+        return rc;
+    NET_TRY(hipMemcpyAsync(dA, a.data(), a.size() * 4, hipMemcpyHostToDevice, d.stream));
+    NET_TRY(hipMemcpyAsync(dW, w.data(), w.size() * 4, hipMemcpyHostToDevice, d.stream));
+    hipLaunchKernelGGL(k_f2bf, dim3(nblk((int64_t)a.size())), dim3(256), 0, d.stream, dA, hA, (int64_t)a.size());
+    PackJobs J{};
+    J.j[0] = PackJob{0, 0, Kp, N, 1, 0};
+    hipLaunchKernelGGL(k_pack, dim3(nblk(nw), 1), dim3(256), 0, d.stream, dW, hW, J);
+    ConvArgs c{};
+    c.in = ConvIn{hA, nullptr, Kp, 0, 0, 1, M};
+    c.Cin = Kp;
+    c.Cout = N;
+    c.ksz = 1;
+    c.sgn = 1;
+    c.Wf = hW;
+    c.Yf = dC;
+    NET_TRY((hipError_t)launch_conv(c, 1, d.stream));
     NET_TRY(hipGetLastError());
-    NET_TRY(hipMemcpy(C, dC, (size_t)M * N * 4, hipMemcpyDeviceToHost));
-    (void)hipFree(dA);
-    (void)hipFree(dB);
-    (void)hipFree(dC);
-    (void)hipFree(hA);
-    (void)hipFree(hB);
+    NET_TRY(hipMemcpyAsync(C, dC, (size_t)M * N * 4, hipMemcpyDeviceToHost, d.stream));
+    NET_TRY(hipStreamSynchronize(d.stream));
     return MTS_OK;
 }
 

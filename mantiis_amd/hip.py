@@ -598,7 +598,7 @@ class Net:
 
 
 def gemm_check(A, B):
-    """C = A B through the network's matrix-core GEMM kernel (BF16 operands)."""
+    """C = A B through the network's convolution kernel (1x1, BF16 operands)."""
     lib = load_library()
     f = C.POINTER(C.c_float)
     lib.mts_net_gemm_check.argtypes = [f, f, C.c_int, C.c_int, C.c_int, f]
