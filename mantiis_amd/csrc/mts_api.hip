@@ -806,8 +806,14 @@ static int create_multi(mts_sim_s* s, int nx, int ny, const int32_t* pore, const
     if (s->prm.precision == MTS_FP32DEV && (rc = create_multi32(s, cr, fr, err))) return rc;
     {
         const size_t np = (size_t)nx * ny;
-        std::vector<uint8_t> lev(np, 0);
-        std::vector<int32_t> site(np, 0);
+        std::vector<uint8_t> lev;
+        std::vector<int32_t> site;
+        try {
+            lev.assign(np, 0);
+            site.assign(np, 0);
+        } catch (...) {
+            return fail(MTS_ERR_OOM, "host allocation");
+        }
         const int nt = np < 65536 ? 1 : host_threads();
         std::atomic<int> next{0};
         on_threads(nt, [&](int) {  // non-buffer cells cover disjoint pixels
@@ -1950,10 +1956,11 @@ int mts_complete_domain(mts_sim s, double* ux, double* uy, double* rho) {
         if (int rc = s->launched()) return rc;
     }
     // the dense site image is row-major and holds 0 at solid sites
-    std::vector<Readback::Piece> pieces;
+    Readback::Piece pieces[Readback::MAX_PIECES];
+    int n = 0;
     for (int k = 0; k < 3; k++)
-        if (outs[k]) pieces.push_back({outs[k], src[k], (size_t)P * 8});
-    HIP_TRY(s->readback.run(s->prm.device, s->stream, pieces));
+        if (outs[k]) pieces[n++] = {outs[k], src[k], (size_t)P * 8};
+    HIP_TRY(s->readback.run(s->prm.device, s->stream, pieces, n));
     return MTS_OK;
 }
 

@@ -12,28 +12,10 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <functional>
-#include <thread>
-#include <vector>
+
+#include "mts_threads.h"
 
 namespace mts {
-
-// Runs work(0) .. work(n - 1) on up to n host threads, the caller's among
-// them.  A thread that cannot be started leaves its share to the others: work
-// items are taken from a common counter by whoever runs.
-inline void on_threads(int n, const std::function<void(int)>& work) {
-    std::vector<std::thread> pool;
-    for (int t = 1; t < n; t++) {
-        try {
-            pool.emplace_back(work, t);
-        } catch (...) {
-            break;
-        }
-    }
-    work(0);
-    for (auto& t : pool) t.join();
-}
-inline int host_threads() { return std::max(1, std::min(8, (int)std::thread::hardware_concurrency())); }
 
 class Readback {
   public:
@@ -42,6 +24,7 @@ class Readback {
         const void* src;
         size_t bytes;
     };
+    static constexpr int MAX_PIECES = 3;
     static constexpr size_t SLOT = (size_t)1 << 20;  // bytes per thread: 8 MB pinned per handle (256 KB slots read at half the rate)
     static constexpr size_t MIN_BYTES = (size_t)24 << 20;  // below, a plain copy costs less than pinning
 
@@ -56,49 +39,48 @@ class Readback {
             failed_ = true;
             return false;
         }
-        ev_.assign(slots_, nullptr);
-        for (hipEvent_t& e : ev_)
-            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        for (int t = 0; t < slots_; t++)
+            if (hipEventCreateWithFlags(&ev_[t], hipEventDisableTiming) != hipSuccess) {
                 (void)hipGetLastError();
-                e = nullptr;
+                ev_[t] = nullptr;
                 release();
                 failed_ = true;
                 return false;
             }
         return true;
     }
-    // Copies the pieces (device to host) behind the work of `stream` and
-    // returns when they are there.
-    hipError_t run(int device, hipStream_t stream, const std::vector<Piece>& pieces) {
-        size_t total = 0;
-        std::vector<size_t> first(1, 0);  // chunks before piece i
-        for (const Piece& p : pieces) {
-            total += p.bytes;
-            first.push_back(first.back() + (p.bytes + SLOT - 1) / SLOT);
+    // Copies n pieces (device to host, at most MAX_PIECES) behind the work of
+    // `stream` and returns when they are there.
+    hipError_t run(int device, hipStream_t stream, const Piece* pieces, int n) noexcept {
+        if (n > MAX_PIECES) return hipErrorInvalidValue;
+        size_t total = 0, first[MAX_PIECES + 1] = {};  // chunks before piece i
+        for (int i = 0; i < n; i++) {
+            total += pieces[i].bytes;
+            first[i + 1] = first[i] + (pieces[i].bytes + SLOT - 1) / SLOT;
         }
         if (total < MIN_BYTES || !ready()) {
-            for (const Piece& p : pieces) {
-                const hipError_t e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+            for (int i = 0; i < n; i++) {
+                const hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes, hipMemcpyDeviceToHost, stream);
                 if (e != hipSuccess) return e;
             }
             return hipStreamSynchronize(stream);
         }
         auto at = [&](size_t c, size_t& i, size_t& off) -> size_t {
-            i = std::upper_bound(first.begin(), first.end(), c) - first.begin() - 1;
+            i = std::upper_bound(first, first + n + 1, c) - first - 1;
             off = (c - first[i]) * SLOT;
             return std::min(SLOT, pieces[i].bytes - off);
         };
         return each(
-            device, stream, first.back(),
+            device, stream, first[n],
             [&](size_t c, char* slot) {
                 size_t i, off;
-                const size_t n = at(c, i, off);
-                return hipMemcpyAsync(slot, (const char*)pieces[i].src + off, n, hipMemcpyDeviceToHost, stream);
+                const size_t len = at(c, i, off);
+                return hipMemcpyAsync(slot, (const char*)pieces[i].src + off, len, hipMemcpyDeviceToHost, stream);
             },
             [&](size_t c, const char* slot) {
                 size_t i, off;
-                const size_t n = at(c, i, off);
-                std::memcpy((char*)pieces[i].dst + off, slot, n);
+                const size_t len = at(c, i, off);
+                std::memcpy((char*)pieces[i].dst + off, slot, len);
             });
     }
     // n chunks on the slots' threads (ready() must hold): fetch(i, slot) queues
@@ -123,9 +105,10 @@ class Readback {
         return (hipError_t)err.load();
     }
     void release() {
-        for (hipEvent_t e : ev_)
+        for (hipEvent_t& e : ev_) {
             if (e) (void)hipEventDestroy(e);
-        ev_.clear();
+            e = nullptr;
+        }
         if (pin_) (void)hipHostFree(pin_);
         pin_ = nullptr;
     }
@@ -133,7 +116,7 @@ class Readback {
 
   private:
     char* pin_ = nullptr;
-    std::vector<hipEvent_t> ev_;
+    hipEvent_t ev_[MAX_HOST_THREADS] = {};
     int slots_ = 0;
     bool failed_ = false;
 };
