@@ -91,7 +91,7 @@ class Readback {
         std::atomic<size_t> next{0};
         std::atomic<int> err{(int)hipSuccess};
         on_threads((int)std::min<size_t>(slots_, n), [&](int t) {
-            hipError_t e = hipSetDevice(device);
+            hipError_t e = t ? hipSetDevice(device) : hipSuccess;  // the caller's thread keeps its current device
             char* slot = pin_ + (size_t)t * SLOT;
             for (size_t c; e == hipSuccess && (c = next.fetch_add(1)) < n;) {
                 e = fetch(c, slot);
