@@ -146,7 +146,7 @@ int launch_cinterface_step(const LaunchCtx& c1, const MbSpec& s1, const LaunchCt
                            const IfSpec& f);
 
 // FP32 production kernels in cell order (mts_compact.inc)
-// The FP32 parameter records (8 floats per (tau_s, Kn) pair) and the SRBB
+// The FP32 parameter records (CPAR_FLOATS per (tau_s, Kn) pair) and the SRBB
 // bookkeeping table (24 floats per pair) of a parameter list.
 void fp32_params(const std::vector<CellParam>& params, double rho0, std::vector<float>& cpar, std::vector<float>& book);
 int launch_ctransport(const LaunchCtx& c, int mode, const TransportSpec& s);

@@ -26,7 +26,13 @@ class Readback {
     };
     static constexpr int MAX_PIECES = 3;
     static constexpr size_t SLOT = (size_t)1 << 20;  // bytes per thread: 8 MB pinned per handle (256 KB slots read at half the rate)
-    static constexpr size_t MIN_BYTES = (size_t)24 << 20;  // below, a plain copy costs less than pinning
+    // Bytes of a lattice's three fields from which they are read through slots:
+    // a handle's 8 MB of pinned memory stay below a third of what it reads with
+    // them.  It is not where the slots begin to pay once they are pinned, which
+    // is at 4 MB (microseconds, plain / slots: 1.6 MB 115 / 140, 3.8 MB 282 / 271,
+    // 6.3 MB 453 / 351, 12 MB 809 / 638, 24.0 MB 1709 / 1196, 25.2 MB 1766 / 1217,
+    // 100 MB 9520 / 3778).
+    static constexpr size_t MIN_BYTES = (size_t)24 << 20;
 
     // Pins the slots (a handle whose fields are large does so when it is made).
     bool ready() {
