@@ -105,14 +105,16 @@ inline size_t conv_lds(int Cin, int ksz, int steps, int rows) {
 // eight channels (the three of the input, the two of the head's gradient) is
 // one step whose eight elements per lane are picked one by one.
 //
-// Bound: the LDS reads of the pixel operand (one 16-byte read per lane feeds
-// NTW products) and the weights' way through the L1 (one read feeds MTW); with
-// offsets, weights and pixels read when they were used, every step waited for
-// the LDS twice: predicting four 512 x 512 images (191 GFLOP) took 767 us
-// against 610 with them read ahead.  The 64x64 implicit GEMM before it, which
+// Bound: latency, with no unit busy (counters: matrix cores 12 to 22% of the
+// time, LDS 8 to 21%; the head 2 to 8%): a block stages its tile and then
+// multiplies, and the accumulators and read-ahead leave two or three waves per
+// SIMD.  With offsets, weights and pixels read when they were used every step
+// also waited for the LDS twice: predicting four 512 x 512 images (191 GFLOP)
+// took 767 us against 605 with them read ahead (one pixel read feeds NTW
+// products, one weight read MTW).  The 64x64 implicit GEMM before it, which
 // fetched every input element nine times through per-element index divisions,
 // took 1703 us; a training step on eight 256 x 256 images went from 5.02 to
-// 2.08 ms with k_convw.
+// 2.00 ms with k_convw.
 // MEM: operands from memory, for tiles that do not fit in LDS.
 template <int MTW, int NTW, int WM, int WN, bool MEM>
 __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
@@ -378,7 +380,9 @@ int launch_conv_t(ConvArgs& a, int B, size_t lds, hipStream_t st) {
 }
 
 // Rows per block: 16 while two blocks fit in a CU's LDS and the launch has at
-// least two blocks per CU; otherwise 8, then 4.
+// least two blocks per CU; otherwise 8, then 4.  The rule looks at LDS only: the
+// 16-row form of six output tiles (more than 80 output channels) takes 308
+// registers, one wave per SIMD, and two of its blocks never share a CU.
 inline int launch_conv(ConvArgs a, int B, hipStream_t st) {
     a.steps = conv_steps(a.Cin, a.ksz);
     constexpr size_t CU_LDS = 160 * 1024;
@@ -484,11 +488,12 @@ __device__ __forceinline__ bf16x8 tr8(const char* p, int stride4) {
 // gradient; channels past the layer's give rows and columns that are not
 // stored.  The bias is the product with a vector of ones.
 //
-// Bound: the LDS reads at few output channels (2 MT / (MT + 3) of a product's
-// operands are reused), staging in between.  The GEMM it replaces gathered the
-// shifted pixels from memory per offset and transposed through 4-byte LDS
-// stores: 118 us per layer on average of a training step on eight 256 x 256
-// images, and a separate 31 us pass for the bias.
+// Bound: the LDS comes nearest at few output channels (33% busy for 24 of them,
+// half of it conflicts; 12 to 15% above; matrix cores 8 to 14%): 2 MT / (MT + 3)
+// of a product's operands are reused, and staging lies between the tiles.  The
+// GEMM it replaces gathered the shifted pixels from memory per offset and
+// transposed through 4-byte LDS stores: 118 us per layer on average of a training
+// step on eight 256 x 256 images (42 now), and a separate 31 us pass for the bias.
 constexpr int WG_H = 8, WG_XS = 80;
 template <int MT>
 __global__ void __launch_bounds__(384) k_convw(WgArgs a) {
